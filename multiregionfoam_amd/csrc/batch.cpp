@@ -361,7 +361,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
                 gm[kBmSteps] = L.waveSteps[w];
                 gm[kBmInbox] = boxIn;
                 gm[kBmSys] = q;
-                boxIn += L.waveSteps[w] * (lm[kBmTB] + kSlice / lm[kBmTB]);
+                boxIn += boxInboxValues(L.waveSteps[w], lm[kBmTB]);
             }
             boxMeta.insert(boxMeta.end(), gm.begin(), gm.end());
         }
@@ -505,9 +505,33 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     for (int w : boxOrder)
         for (int k : {kBmPrevB, kBmPrevC, kBmNextB, kBmNextC})
             if (boxMeta[(size_t)w * kBoxMeta + k] >= 0) boxLone_ = false;
+    std::vector<int32_t> boxTile;
+    for (int w : boxOrder) {
+        const int32_t *g = &boxMeta[(size_t)w * kBoxMeta];
+        std::array<int32_t, kBoxTile> t{};
+        t[kBtTB] = g[kBmTB];
+        t[kBtNA] = g[kBmNA];
+        t[kBtAxis] = g[kBmAxis];
+        t[kBtActB] = g[kBmActB];
+        t[kBtActC] = g[kBmActC];
+        t[kBtSlice] = g[kBmSlice];
+        t[kBtSteps] = g[kBmSteps];
+        t[kBtSys] = g[kBmSys];
+        t[kBtInbox] = g[kBmInbox];
+        const int side[4] = {kBmPrevB, kBmPrevC, kBmNextB, kBmNextC};
+        for (int k = 0; k < 4; ++k) {
+            t[kBtInPrevB + k] = -1;
+            if (g[side[k]] < 0) continue;
+            const int32_t *n = &boxMeta[(size_t)g[side[k]] * kBoxMeta];
+            t[kBtInPrevB + k] = n[kBmInbox];
+            t[kBtLPrevB + k] = n[kBmSteps];
+        }
+        boxTile.insert(boxTile.end(), t.begin(), t.end());
+    }
     if (nGenWaves_ == 0) nHaloF_ = nHaloB_ = 0;
     if (order.empty()) order.push_back(0);
     if (boxOrder.empty()) boxOrder.push_back(0);
+    if (boxTile.empty()) boxTile.push_back(0);
 
     hipStream_t st = stream_;
     ellOff_.upload(ellOff, st);
@@ -546,6 +570,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     boxOrder_.upload(boxOrder, st);
     waveOut_.upload(waveOut, st);
     boxMeta_.upload(boxMeta, st);
+    boxTile_.upload(boxTile, st);
     waveSlice_.upload(waveSlice, st);
     waveSteps_.upload(waveSteps, st);
     waveSys_.upload(waveSys, st);
@@ -673,6 +698,7 @@ DiluView<T> Batch::diluView(DevMatrix<T> &m, void *hF, void *hB)
     D.boxLone = boxLone_ || local;
     D.boxSegs = local ? tileSegments() : 1;
     D.boxMeta = boxMeta_.p;
+    D.boxTile = boxTile_.p;
     D.nBoxIn = nBoxIn_;
     D.fCodes = fCodes_.p;
     D.waveOut = waveOut_.p;

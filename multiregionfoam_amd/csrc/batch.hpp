@@ -390,7 +390,7 @@ private:
     void launchCfg(int slices, const BlockEntry *&blocks, int &nBlk, const SysInfo *&info, int &threads) const;
     void setTuning(int slices, int ellChunk);
     // DILU schedule
-    DevBuf<int32_t> order_, waveSlice_, waveSteps_, waveSys_, waveOut_, boxOrder_, boxMeta_;
+    DevBuf<int32_t> order_, waveSlice_, waveSteps_, waveSys_, waveOut_, boxOrder_, boxMeta_, boxTile_;
     std::vector<int32_t> hBoxMeta_, hBoxWaves_;   // host copies: box tile geometry, the box waves
     DevBuf<double> rdLocal_;                      // rD of the tile-local factor
     DevBuf<unsigned long long> rowMask_;   // per slice: lanes holding a cell

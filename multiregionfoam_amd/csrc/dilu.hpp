@@ -70,9 +70,9 @@ struct DiluView {
     void *haloF = nullptr, *haloB = nullptr, *haloC = nullptr;   // inboxes
     int nHaloF = 0, nHaloB = 0;          // inbox sizes (values)
     int *err = nullptr;                  // bit 2: a halo wait expired
-    // structured-box tile waves (dilu.hip, k_dilu_box): their own dispatch
-    // order, kBoxMeta ints of tile geometry per wave, and compact inboxes of
-    // (TB + TC) values per step per wave, one per direction
+    // structured-box tiles (dilu_box.hip; the factor in dilu.hip): their own
+    // dispatch order, kBoxMeta ints of tile geometry per wave, and compact
+    // inboxes of 2 max(TB, TC) values per step per tile, one per direction
     const int32_t *boxOrder = nullptr;
     int nBoxWaves = 0;
     bool boxLone = false;                // every box tile is alone in its region
@@ -82,6 +82,7 @@ struct DiluView {
     // left out
     int boxSegs = 1;
     const int32_t *boxMeta = nullptr;
+    const int32_t *boxTile = nullptr;    // kBoxTile ints per box tile, in dispatch order
     void *boxInF = nullptr, *boxInB = nullptr, *boxInC = nullptr;
     int nBoxIn = 0;
     // optional trace: per wave start / end realtime clock ticks, slow-path
@@ -111,6 +112,11 @@ struct SweepInput {
 
 // Forward sweep out = (D+L)^-1 in (with the D^-1 scaling of DILU) and the
 // backward sweep in place; systems whose status is not running are skipped.
+// the box tiles alone (dilu_box.hip)
+template <typename T>
+hipError_t boxForward(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s);
+template <typename T>
+hipError_t boxBackward(const DiluView<T> &V, const SysState *st, T *inout, hipStream_t s);
 template <typename T>
 hipError_t diluForward(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s);
 template <typename T>
@@ -147,6 +153,18 @@ __host__ __device__ inline void boxSegment(int nA, int s, int segs, int &lo, int
     lo = (int)((long long)s * nA / segs);
     hi = (int)((long long)(s + 1) * nA / segs);
 }
+// Values of a box tile's inbox: per step one row for the b and one for the c edge
+__host__ __device__ inline int boxInboxValues(int nSteps, int TB) { return nSteps * 2 * (TB > 64 / TB ? TB : 64 / TB); }
+
+// A box tile as its sweeps see it: one descriptor per tile in forward
+// dispatch order (the backward sweep takes them in reverse), with the inbox
+// of every neighbouring tile (-1: none) and the steps of the next ones, so a
+// workgroup starts after two dependent loads
+enum {
+    kBtTB = 0, kBtNA, kBtAxis, kBtActB, kBtActC, kBtSlice, kBtSteps, kBtSys, kBtInbox,
+    kBtInPrevB, kBtInPrevC, kBtInNextB, kBtInNextC, kBtLPrevB, kBtLPrevC, kBtLNextB, kBtLNextC,
+    kBoxTile = 20
+};
 // rD of the FP32 records from the FP64 factor
 hipError_t diluConvertRD(const DiluView<float> &V32, const double *rD64, int nSlices, hipStream_t s);
 hipError_t fillHalo64(void *h, int n, hipStream_t s);

@@ -1,0 +1,52 @@
+"""DILU sweeps of structured boxes against the oracle, bit for bit, over the
+shapes where a tile's schedule changes: tiles of every width the schedule
+picks, partial tiles on either edge, lines shorter than a group of steps,
+every sequential axis, boxes of one tile and of many, a single row of cells."""
+import numpy as np
+import pytest
+
+import oracle_bind as ob
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(3, 2, 2), (40, 1, 1), (7, 5, 1), (64, 64, 1), (200, 130, 1), (11, 9, 5), (33, 17, 9), (17, 33, 70),
+          (20, 90, 31), (90, 66, 3), (150, 40, 40)]
+
+
+def box(n, seed, symmetric=False):
+    """Random diagonally dominant matrix on the faces of an n box."""
+    rng = np.random.default_rng(seed)
+    N = int(np.prod(n))
+    c = np.arange(N)
+    ijk = (c % n[0], (c // n[0]) % n[1], c // (n[0] * n[1]))
+    has = np.stack([ijk[a] + 1 < n[a] for a in range(3)], axis=1)
+    cell, axis = np.nonzero(has)
+    nb = cell + np.take((1, n[0], n[0] * n[1]), axis)
+    upper = -rng.uniform(0.1, 2.0, len(cell))
+    lower = upper.copy() if symmetric else -rng.uniform(0.1, 2.0, len(cell))
+    diag = 0.3 - np.bincount(cell, upper, N) - np.bincount(nb, lower, N)
+    return dict(nCells=N, nFaces=len(cell), symmetric=symmetric, lAddr=cell.astype(np.int32),
+                uAddr=nb.astype(np.int32), lower=lower, upper=upper, diag=diag, source=rng.standard_normal(N),
+                psi=rng.standard_normal(N))
+
+
+@pytest.mark.parametrize("n", SHAPES, ids=lambda n: "x".join(map(str, n)))
+def test_sweeps_match_oracle(gpu, n):
+    # two boxes in one system, so that tiles of both are swept by one launch
+    regions = [box(n, 1), box((n[0], n[2], n[1]), 2, symmetric=True)]
+    O = ob.OracleSystem.from_arrays(regions, [])
+    A = gpu.CoupledFvMatrix(0)
+    A.add_system(regions, [])
+    A.commit()
+    rD = O.dilu_factor()
+    assert np.array_equal(A.dilu_factor(), np.concatenate(rD))
+    rng = np.random.default_rng(3)
+    for _ in range(2):
+        r = [rng.standard_normal(R["nCells"]) for R in regions]
+        assert np.array_equal(A.precondition(r), np.concatenate(O.dilu_precondition(rD, r)))
+    # the fused p and s updates, in a solve that starts and ends on its own
+    psi, perf = O.solve(tol=1e-10, maxIter=40)
+    got = A.solve(tolerance=1e-10, maxIter=40)[0]
+    assert got.n_iterations == perf["nIterations"] and got.final_residual == perf["finalResidual"]
+    assert np.array_equal(np.concatenate(A.psi(0)), np.concatenate(psi))
+    A.close()
