@@ -66,6 +66,8 @@ template struct DevBuf<float>;
 template struct DevBuf<int32_t>;
 template struct DevBuf<unsigned long long>;
 template struct DevBuf<int8_t>;
+template struct DevBuf<LevelGroup>;
+template struct DevBuf<int2>;
 template struct DevBuf<FvRegionParams>;
 template struct DevBuf<DnaSide>;
 template struct DevBuf<DnaCell>;
@@ -268,7 +270,8 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
 
     std::vector<int32_t> ellOff, ellCol, ifBase, ifRowFace, ifPairOff, ifPairCol;
     std::vector<unsigned long long> ifMask;
-    std::vector<int32_t> cellOfPos, fCode, bCode, fHalo, bHalo, waveSlice, waveSteps, waveSys, waveOut;
+    std::vector<int32_t> cellOfPos, fCode, bCode, waveSlice, waveSteps, waveSys;
+    std::vector<const std::vector<int32_t> *> waveLevels;
     std::vector<double> diag, source, sumA, psi0, fProd;
     std::vector<std::array<int, 3>> waveKey;   // (key, system, global wave index)
     std::vector<uint8_t> waveBox;
@@ -280,7 +283,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     std::vector<double> ddtA, diagBase, srcBase;
     bool anyTransient = false;
 
-    int slice = 0, ellBase = 0, ifRowBase = 0, ifFaceBase = 0, ifPairBase = 0, hfBase = 0, hbBase = 0;
+    int slice = 0, ellBase = 0, ifRowBase = 0, ifFaceBase = 0, ifPairBase = 0;
     for (int q = 0; q < nS; ++q) {
         const SystemLayout &L = *lay_[q];
         const int pos0 = slice * kSlice;
@@ -317,16 +320,14 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
         hEllVal_.insert(hEllVal_.end(), L.ellVal.begin(), L.ellVal.end());
         hIfCoeff_.insert(hIfCoeff_.end(), L.ifCoeff.begin(), L.ifCoeff.end());
         hIfPairW_.insert(hIfPairW_.end(), L.ifPairW.begin(), L.ifPairW.end());
-        // DILU dependency slots, re-padded to the batch width K_; halo codes
-        // and halo slots are shifted to the system's halo range
+        // DILU dependency slots, re-padded to the batch width K_
         for (int s = 0; s < L.nSlices; ++s)
             for (int k = 0; k < K_; ++k)
                 for (int l = 0; l < kSlice; ++l) {
                     if (k < L.K) {
                         size_t e = ((size_t)s * L.K + k) * kSlice + l;
-                        int fc = L.fCode[e], bc = L.bCode[e];
-                        fCode.push_back(fc >= 0 ? fc + hfBase : fc);
-                        bCode.push_back(bc >= 0 ? bc + hbBase : bc);
+                        fCode.push_back(L.fCode[e]);
+                        bCode.push_back(L.bCode[e]);
                         hFVal_.push_back(L.fVal[e]);
                         hBVal_.push_back(L.bVal[e]);
                         fProd.push_back(L.fProd[e]);
@@ -338,10 +339,6 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
                         fProd.push_back(0.0);
                     }
                 }
-        for (int p = 0; p < L.nPos; ++p) {
-            fHalo.push_back(L.fHalo[p] >= 0 ? L.fHalo[p] + hfBase : -1);
-            bHalo.push_back(L.bHalo[p] >= 0 ? L.bHalo[p] + hbBase : -1);
-        }
         SysInfo &I = hInfo_[q];
         I.waveBegin = (int)waveSlice.size();
         for (int w = 0; w < L.nWaves; ++w) {
@@ -350,6 +347,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
             waveSteps.push_back(L.waveSteps[w]);
             waveSys.push_back(q);
             waveBox.push_back(L.waveBox[w]);
+            waveLevels.push_back(&L.waveLevels[w]);
             // box tile geometry with batch-wide wave, slice and inbox indices
             const int32_t *lm = &L.boxMeta[(size_t)w * kBoxMeta];
             std::array<int32_t, kBoxMeta> gm;
@@ -379,106 +377,63 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
         ifRowBase += (int)L.ifRowFace.size() - 1;
         ifFaceBase += (int)L.ifCoeff.size();
         ifPairBase += (int)L.ifPairW.size();
-        hfBase += L.nHaloF;
-        hbBase += L.nHaloB;
     }
     ellOff.push_back(ellBase);
     ifRowFace.push_back(ifFaceBase);
     // pack the DILU records: values [c_0..c_{K-1}, rD | diag] in chunks of
-    // Pack<T>::N; ints [byte codes, out_0..out_{K-1}] in chunks of 4.  A
-    // cross-wave dependency is delivered to the consumer's inbox slot
-    // (slice, kk, lane); its producer's outs list those inbox addresses.
+    // Pack<T>::N, and the codes of the general waves
     {
         const int nSl = slice;
-        const int G = packChunks(K_ + 1, 2);
-        const int NC = packChunks(K_, 4), H = packChunks(codeInts(K_), 4);
-        int rawF = 0, rawB = 0;
-        for (size_t e = 0; e < fCode.size(); ++e) {
-            if (fCode[e] >= 0) rawF |= 1 << (int)((e / kSlice) % K_);
-            if (bCode[e] >= 0) rawB |= 1 << (int)((e / kSlice) % K_);
-        }
-        haloMaskF_ = rawF;
-        haloMaskB_ = rawB;
-        const int mF = effectiveHaloMask(K_, rawF), mB = effectiveHaloMask(K_, rawB);
-        const int KIF = __builtin_popcount(mF), KIB = __builtin_popcount(mB);
-        auto kkOf = [](int m, int k) { return __builtin_popcount(m & ((1 << k) - 1)); };
+        const int G = packChunks(K_ + 1, 2), NC = packChunks(K_, 4);
         hFPack_.assign((size_t)nSl * G * 64 * 2, 0.0);
         hBPack_.assign((size_t)nSl * G * 64 * 2, 0.0);
         hFPack32_.clear();   // derived from the FP64 records when mixed precision first needs them
         hBPack32_.clear();
         std::vector<double> prod((size_t)nSl * G * 64 * 2, 0.0);
-        std::vector<int32_t> fc((size_t)nSl * H * 64 * 4, -1), bc((size_t)nSl * H * 64 * 4, -1);
-        // consumers of every published halo value (slot id -> inbox addresses)
-        std::vector<std::vector<int32_t>> fOuts(hfBase), bOuts(hbBase);
-        auto intAt = [&](int s, int j, int l) { return (((size_t)s * H + j / 4) * 64 + l) * 4 + j % 4; };
         for (int s = 0; s < nSl; ++s)
             for (int l = 0; l < kSlice; ++l) {
-                const int p = s * kSlice + l;
-                uint32_t fw[4] = {0, 0, 0, 0}, bw[4] = {0, 0, 0, 0};
                 for (int k = 0; k < K_; ++k) {
                     size_t e = ((size_t)s * K_ + k) * kSlice + l;
-                    auto byteOf = [&](int code, int mask, int KI, std::vector<std::vector<int32_t>> &outs) {
-                        if (code == kNoDep) return kCodeNone;
-                        if (code < 0) return -code - 1;            // LDS ring slot
-                        if (!(mask & (1 << k))) throw std::runtime_error("DILU inbox mask misses a dependency slot");
-                        outs[code].push_back(((s * KI + kkOf(mask, k)) << 6) + l);
-                        return kCodeInbox;
-                    };
-                    uint32_t fb = (uint32_t)byteOf(fCode[e], mF, KIF, fOuts);
-                    uint32_t bb = (uint32_t)byteOf(bCode[e], mB, KIB, bOuts);
-                    fw[k / 4] |= fb << (8 * (k % 4));
-                    bw[k / 4] |= bb << (8 * (k % 4));
                     size_t e64 = (((size_t)s * G + k / 2) * 64 + l) * 2 + k % 2;
                     hFPack_[e64] = hFVal_[e];
                     hBPack_[e64] = hBVal_[e];
                     prod[e64] = fProd[e];
                 }
-                // padding slots of the last code int are "none"
-                for (int k = K_; k < NC * 4; ++k) {
-                    fw[k / 4] |= (uint32_t)kCodeNone << (8 * (k % 4));
-                    bw[k / 4] |= (uint32_t)kCodeNone << (8 * (k % 4));
-                }
-                for (int j = 0; j < NC; ++j) {
-                    fc[intAt(s, j, l)] = (int32_t)fw[j];
-                    bc[intAt(s, j, l)] = (int32_t)bw[j];
-                }
-                prod[(((size_t)s * G + K_ / 2) * 64 + l) * 2 + K_ % 2] = diag[p];
+                prod[(((size_t)s * G + K_ / 2) * 64 + l) * 2 + K_ % 2] = diag[s * kSlice + l];
             }
-        for (int s = 0; s < nSl; ++s)
-            for (int l = 0; l < kSlice; ++l) {
-                const int p = s * kSlice + l;
-                auto putOuts = [&](int h, std::vector<std::vector<int32_t>> &outs, std::vector<int32_t> &dst) {
-                    if (h < 0) return;
-                    if ((int)outs[h].size() > K_) throw std::runtime_error("DILU value has more consumers than slots");
-                    for (size_t j = 0; j < outs[h].size(); ++j) dst[intAt(s, NC + (int)j, l)] = outs[h][j];
-                };
-                putOuts(fHalo[p], fOuts, fc);
-                putOuts(bHalo[p], bOuts, bc);
-            }
-        // per wave: bit 0 (1) when a row of it delivers a forward (backward)
-        // value to another wave's inbox; a wave without skips the deliveries
-        waveOut.assign(waveSlice.size(), 0);
+        // a chain's codes as bytes; a level group's as they are
+        bool chains = false, groups = false;
         for (size_t w = 0; w < waveSlice.size(); ++w)
-            for (int s = waveSlice[w]; s < waveSlice[w] + waveSteps[w]; ++s)
-                for (int l = 0; l < kSlice; ++l)
-                    for (int j = 0; j < K_; ++j) {
-                        if (fc[intAt(s, NC + j, l)] >= 0) waveOut[w] |= 1;
-                        if (bc[intAt(s, NC + j, l)] >= 0) waveOut[w] |= 2;
-                    }
-        nHaloF_ = nSl * KIF * 64;
-        nHaloB_ = nSl * KIB * 64;
-        auto asVec = [](const std::vector<int32_t> &a) {
-            std::vector<int4> v(a.size() / 4);
-            std::memcpy(v.data(), a.data(), a.size() * sizeof(int32_t));
+            if (!waveBox[w]) (waveLevels[w]->empty() ? chains : groups) = true;
+        auto bytes = [&](const std::vector<int32_t> &code) {
+            std::vector<int32_t> v(chains ? (size_t)nSl * NC * 64 : 1, -1);
+            if (!chains) return v;
+            for (size_t w = 0; w < waveSlice.size(); ++w) {
+                if (waveBox[w] || !waveLevels[w]->empty()) continue;
+                for (int s = waveSlice[w]; s < waveSlice[w] + waveSteps[w]; ++s)
+                    for (int l = 0; l < kSlice; ++l)
+                        for (int j = 0; j < NC; ++j) {
+                            uint32_t x = 0xFFFFFFFFu;
+                            for (int k = 4 * j; k < std::min(4 * j + 4, K_); ++k) {
+                                const int32_t q = code[((size_t)s * K_ + k) * kSlice + l];
+                                const uint32_t byte = q == kNoDep ? kCodeNone : (uint32_t)q;
+                                x = (x & ~(0xFFu << (8 * (k % 4)))) | byte << (8 * (k % 4));
+                            }
+                            v[((size_t)s * NC + j) * 64 + l] = (int32_t)x;
+                        }
+            }
             return v;
         };
+        fCodes_.upload(bytes(fCode), stream_);
+        bCodes_.upload(bytes(bCode), stream_);
+        fDeps_.upload(groups ? fCode : std::vector<int32_t>(1, kNoDep), stream_);
+        bDeps_.upload(groups ? bCode : std::vector<int32_t>(1, kNoDep), stream_);
+        lvD_.alloc(groups ? (size_t)nSl * 64 : 1);
         auto asD2 = [](const std::vector<double> &a) {
             std::vector<double2> v(a.size() / 2);
             std::memcpy(v.data(), a.data(), a.size() * sizeof(double));
             return v;
         };
-        fCodes_.upload(asVec(fc), stream_);
-        bCodes_.upload(asVec(bc), stream_);
         prodPack_.upload(asD2(prod), stream_);
         m64_.fPack.upload(asD2(hFPack_), stream_);
         m64_.bPack.upload(asD2(hBPack_), stream_);
@@ -489,13 +444,45 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     nBlk_ = (int)blocks.size();
     nWaves_ = (int)waveSlice.size();
 
-    // forward dispatch order: by key (tile anti-diagonal / level), systems
-    // interleaved; every wave's producers precede it.  Box tile waves and
-    // general waves never depend on each other (DILU dependencies stay inside
+    // forward dispatch order: by key (tile anti-diagonal), systems
+    // interleaved; every tile's producers precede it.  Box tiles, chains and
+    // level groups never depend on each other (DILU dependencies stay inside
     // a region) and run in kernels of their own.
     std::sort(waveKey.begin(), waveKey.end());
     std::vector<int32_t> order, boxOrder;
-    for (int i = 0; i < nWaves_; ++i) (waveBox[waveKey[i][2]] ? boxOrder : order).push_back(waveKey[i][2]);
+    std::vector<int> grouped;
+    for (int i = 0; i < nWaves_; ++i) {
+        const int w = waveKey[i][2];
+        if (waveBox[w]) boxOrder.push_back(w);
+        else if (waveLevels[w]->empty()) order.push_back(w);
+        else grouped.push_back(w);
+    }
+    // level groups: rounds of as many slices of one level as a workgroup has
+    // waves (as many as the widest level needs, at most 16)
+    int widest = 1;
+    for (int w : grouped)
+        for (int n : *waveLevels[w]) widest = std::max(widest, n);
+    lvWaves_ = std::min(16, widest);
+    lvDrain_ = widest * kSlice > kLevelRing / 4;
+    std::vector<LevelGroup> groups;
+    std::vector<int2> rounds;
+    for (int w : grouped) {
+        LevelGroup g{waveSlice[w], (int)rounds.size(), 0, waveSys[w]};
+        int s = waveSlice[w];
+        for (int n : *waveLevels[w])
+            for (int k = 0; k < n; k += lvWaves_) {
+                const int cnt = std::min(lvWaves_, n - k);
+                rounds.push_back(int2{s, cnt << 2 | (k + cnt == n ? kRoundLast : 0) | (k == 0 ? kRoundFirst : 0)});
+                s += cnt;
+            }
+        g.nRounds = (int)rounds.size() - g.round0;
+        groups.push_back(g);
+    }
+    nGroups_ = (int)groups.size();
+    if (groups.empty()) groups.push_back(LevelGroup{});
+    if (rounds.empty()) rounds.push_back(int2{0, 0});
+    groups_.upload(groups, stream_);
+    lvRounds_.upload(rounds, stream_);
     nGenWaves_ = (int)order.size();
     nBoxWaves_ = (int)boxOrder.size();
     nBoxIn_ = boxIn;
@@ -528,7 +515,6 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
         }
         boxTile.insert(boxTile.end(), t.begin(), t.end());
     }
-    if (nGenWaves_ == 0) nHaloF_ = nHaloB_ = 0;
     if (order.empty()) order.push_back(0);
     if (boxOrder.empty()) boxOrder.push_back(0);
     if (boxTile.empty()) boxTile.push_back(0);
@@ -568,16 +554,14 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     tune_ = Tuning{};
     order_.upload(order, st);
     boxOrder_.upload(boxOrder, st);
-    waveOut_.upload(waveOut, st);
     boxMeta_.upload(boxMeta, st);
     boxTile_.upload(boxTile, st);
     waveSlice_.upload(waveSlice, st);
     waveSteps_.upload(waveSteps, st);
     waveSys_.upload(waveSys, st);
-    // each inbox buffer: general part, then the box part
-    haloF64_.alloc(std::max(1, nHaloF_ + nBoxIn_));
-    haloB64_.alloc(std::max(1, nHaloB_ + nBoxIn_));
-    haloC64_.alloc(std::max(1, nHaloF_ + nBoxIn_));
+    haloF64_.alloc(std::max(1, nBoxIn_));
+    haloB64_.alloc(std::max(1, nBoxIn_));
+    haloC64_.alloc(std::max(1, nBoxIn_));
     HIP_OK(fillHalo64(haloF64_.p, (int)haloF64_.n, st));
     HIP_OK(fillHalo64(haloB64_.p, (int)haloB64_.n, st));
     HIP_OK(fillHalo64(haloC64_.p, (int)haloC64_.n, st));
@@ -652,8 +636,8 @@ void Batch::ensureFloat(bool tileLocal)
         v.alloc(nPos_);
         v.zero(st);
     }
-    haloF32_.alloc(std::max(1, nHaloF_ + nBoxIn_));
-    haloB32_.alloc(std::max(1, nHaloB_ + nBoxIn_));
+    haloF32_.alloc(std::max(1, nBoxIn_));
+    haloB32_.alloc(std::max(1, nBoxIn_));
     HIP_OK(fillHalo32(haloF32_.p, (int)haloF32_.n, st));
     HIP_OK(fillHalo32(haloB32_.p, (int)haloB32_.n, st));
     haveFloat_ = true;
@@ -701,23 +685,23 @@ DiluView<T> Batch::diluView(DevMatrix<T> &m, void *hF, void *hB)
     D.boxTile = boxTile_.p;
     D.nBoxIn = nBoxIn_;
     D.fCodes = fCodes_.p;
-    D.waveOut = waveOut_.p;
     D.bCodes = bCodes_.p;
     D.fPack = m.fPack.p;
     D.bPack = m.bPack.p;
     D.prodPack = prodPack_.p;
     D.rDout = v64_[11].p;
     D.cellOfPos = cellOfPos_.p;
-    D.haloMaskF = haloMaskF_;
-    D.haloMaskB = haloMaskB_;
-    D.haloF = hF;
-    D.haloB = hB;
-    D.haloC = haloC64_.p;
-    D.nHaloF = nHaloF_;
-    D.nHaloB = nHaloB_;
-    D.boxInF = (char *)hF + (size_t)nHaloF_ * sizeof(T);
-    D.boxInB = (char *)hB + (size_t)nHaloB_ * sizeof(T);
-    D.boxInC = (char *)haloC64_.p + (size_t)nHaloF_ * sizeof(double);
+    D.groups = groups_.p;
+    D.lvRounds = lvRounds_.p;
+    D.fDeps = fDeps_.p;
+    D.bDeps = bDeps_.p;
+    D.nGroups = nGroups_;
+    D.lvWaves = lvWaves_;
+    D.lvDrain = lvDrain_;
+    D.lvD = lvD_.p;
+    D.boxInF = hF;
+    D.boxInB = hB;
+    D.boxInC = haloC64_.p;
     D.err = err_.p;
     D.side = side_;
     D.fork = fork_;

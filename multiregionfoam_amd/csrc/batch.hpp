@@ -353,7 +353,7 @@ private:
     std::vector<std::unique_ptr<SystemLayout>> lay_;
     std::vector<const CoupledSystem *> sys_;
     std::vector<int> sliceBegin_;
-    int nSlices_ = 0, nPos_ = 0, nBlk_ = 0, nWaves_ = 0, K_ = 3, nHaloF_ = 0, nHaloB_ = 0;
+    int nSlices_ = 0, nPos_ = 0, nBlk_ = 0, nWaves_ = 0, K_ = 3;
     int nGenWaves_ = 0, nBoxWaves_ = 0, nBoxIn_ = 0;
     bool boxLone_ = false;   // every box tile alone in its region
     bool factorised_ = false, haveFloat_ = false;
@@ -390,13 +390,17 @@ private:
     void launchCfg(int slices, const BlockEntry *&blocks, int &nBlk, const SysInfo *&info, int &threads) const;
     void setTuning(int slices, int ellChunk);
     // DILU schedule
-    DevBuf<int32_t> order_, waveSlice_, waveSteps_, waveSys_, waveOut_, boxOrder_, boxMeta_, boxTile_;
+    DevBuf<int32_t> order_, waveSlice_, waveSteps_, waveSys_, boxOrder_, boxMeta_, boxTile_;
     std::vector<int32_t> hBoxMeta_, hBoxWaves_;   // host copies: box tile geometry, the box waves
     DevBuf<double> rdLocal_;                      // rD of the tile-local factor
     DevBuf<unsigned long long> rowMask_;   // per slice: lanes holding a cell
-    DevBuf<int4> fCodes_, bCodes_;
+    DevBuf<int32_t> fCodes_, bCodes_, fDeps_, bDeps_;
+    DevBuf<LevelGroup> groups_;
+    DevBuf<int2> lvRounds_;
+    DevBuf<double> lvD_;                          // d of the level groups' rows (factor)
+    int nGroups_ = 0, lvWaves_ = 1;
+    bool lvDrain_ = false;
     DevBuf<double2> prodPack_;
-    int haloMaskF_ = 0, haloMaskB_ = 0;
     DevBuf<unsigned long long> haloF64_, haloB64_, haloC64_;
     DevBuf<unsigned int> haloF32_, haloB32_;
     DevBuf<int> err_;

@@ -8,20 +8,16 @@
 //   forward   w[u] = rD[u]*r[u] - sum_{lower faces, face order} rD[u]*lower_f*w[l(f)]
 //   backward  w[l] -= sum_{upper faces, reverse face order} rD[l]*upper_f*w[u(f)]
 //
-// Each lane holds one row per step.  A dependency produced by the same wave
-// at most kRing-1 steps earlier is read from the wave's LDS ring; any other
-// is read from a halo slot that its producer stores with a relaxed
-// agent-scope atomic.  Halo buffers are reset to a sentinel bit pattern
-// before a sweep (by the previous sweep), so a consumer simply polls the
-// slot until the value differs from the sentinel: no fences, no counters.
-// Every wait is bounded; an expired wait raises the error flag.
+// General regions only: the sweeps of structured boxes are in dilu_box.hip,
+// their factorisation at the end of this file.
 //
-// A step is latency-bound (one LDS round trip plus a short FMA chain), so
-// the kernel keeps memory out of the critical path: each row's record is a
-// few 16-byte chunks, records and inbox values are prefetched kPrefetch
-// steps ahead, every prefetch load is unconditional (the
-// compiler then counts outstanding loads exactly instead of draining them),
-// and the fast path has no divergent branch.
+// Each lane holds one row per step, whose dependencies were computed earlier
+// by the same wave (chains) or workgroup (level groups) and are read from LDS.
+// A step of a chain is latency-bound (one LDS round trip plus a short FMA
+// chain), so the kernel keeps memory out of the critical path: each row's
+// record is a few 16-byte chunks, prefetched kPrefetch steps ahead, every
+// prefetch load is unconditional (the compiler then counts outstanding loads
+// exactly instead of draining them), and the fast path has no divergent branch.
 #include <hip/hip_runtime.h>
 #include <type_traits>
 
@@ -38,105 +34,74 @@ static_assert(kWaveGroup % kRing == 0, "a group of steps spans whole rounds of t
 // LDS values of a wave's ring: kRing steps, then zeros up to the largest
 // code byte, so that every code byte indexes the ring
 constexpr int kRingSlots = 256;
-static_assert(kRing * 64 <= kCodeInbox, "ring slots lie below the reserved code bytes");
-
-template <typename U>
-__device__ inline U haloWait(const U *h, int slot, U sent, int *err)
-{
-    U v = haloLoad(h, slot);
-    int spins = 0;
-    while (v == sent) {
-        // once any wait has expired every later one gives up at once, so a
-        // broken schedule ends the kernel quickly instead of hanging it
-        if (++spins > kPollLimit || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-            atomicOr(err, 2);
-            break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-        v = haloLoad(h, slot);
-    }
-    return v;
-}
+static_assert(kRing * 64 <= kCodeNone, "ring slots lie below the reserved code byte");
 
 }  // namespace
 
+// A chain: one wave whose steps are the region's levels.
 // MODE: kDiluFwd / kDiluBwd (T = value type) or kDiluFactor (T = double).
-// HMASK: dependency slots that have an inbox (compile-time, so all inbox
-// prefetch loads are unconditional code).
-template <typename T, int K, int MODE, int HMASK>
-__global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState *st, const T *__restrict__ in,
-                                                  T *out, typename Bits<T>::U *inbox,
-                                                  typename Bits<T>::U *inboxClear, int nClear)
+template <typename T, int K, int MODE>
+__global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState *st, const T *in, T *out)
 {
-    using U = typename Bits<T>::U;
     using R = typename RecordOf<T, MODE>::V;
     constexpr int N = RecordOf<T, MODE>::N;
     constexpr int G = packChunks(K + 1, N);      // value chunks per row
     constexpr int NC = packChunks(K, 4);         // ints holding the byte codes
-    constexpr int H = packChunks(codeInts(K), 4);
-    constexpr int KI = __builtin_popcount(HMASK);
-    constexpr U kSent = Bits<T>::kSent;
     __shared__ T ring[kRingSlots];
     const int lane = threadIdx.x;
     const int w = MODE == kDiluBwd ? V.order[V.nWaves - 1 - blockIdx.x] : V.order[blockIdx.x];
     const int sys = V.waveSys[w];
     const bool active = MODE == kDiluFactor || st[sys].status == kRunning;
     const int s0 = V.waveSlice[w], nSteps = V.waveSteps[w];
-    const int4 *codes = MODE == kDiluBwd ? V.bCodes : V.fCodes;
-    // whether any row of this wave delivers to another wave (wave-uniform)
-    const bool delivers = (V.waveOut[w] & (MODE == kDiluBwd ? 2 : 1)) != 0;
+    const int32_t *codes = MODE == kDiluBwd ? V.bCodes : V.fCodes;
     const R *recs = MODE == kDiluFactor ? (const R *)V.prodPack : (const R *)(MODE == kDiluBwd ? V.bPack : V.fPack);
     const unsigned long long tStart = V.trace ? wall_clock64() : 0ull;
-    unsigned long long nSlow = 0;
 
     struct Step {
         R v[G];
-        int4 c[H];
-        U hv[KI > 0 ? KI : 1];
+        int c[NC];
         T a;
     };
     auto sliceOf = [&](int i) {
         i = i < nSteps ? i : nSteps - 1;
         return s0 + (MODE == kDiluBwd ? nSteps - 1 - i : i);
     };
-    // the row's record, input and inbox values, kPrefetch steps ahead.  Every
-    // address is computable without another load, and steps past the end
-    // re-read the last step, so no load waits for another or is conditional.
+    // the row's record and input, kPrefetch steps ahead.  Every address is
+    // computable without another load, and steps past the end re-read the
+    // last step, so no load waits for another or is conditional.
     auto load = [&](int i, Step &S) {
         const int s = sliceOf(i);
 #pragma unroll
         for (int g = 0; g < G; ++g) S.v[g] = recs[((size_t)s * G + g) * 64 + lane];
 #pragma unroll
-        for (int h = 0; h < H; ++h) S.c[h] = codes[((size_t)s * H + h) * 64 + lane];
-#pragma unroll
-        for (int kk = 0; kk < KI; ++kk) S.hv[kk] = haloLoad(inbox, ((s * KI + kk) << 6) + lane);
+        for (int h = 0; h < NC; ++h) S.c[h] = codes[((size_t)s * NC + h) * 64 + lane];
         if (MODE != kDiluFactor) S.a = in[s * 64 + lane];
     };
 
     // FULL groups (below) address a step through per-wave resources: the
     // wave's rows of the records, codes, input and output, a scalar offset of
     // the step's slice in the wave and a per-lane constant
-    constexpr bool kCanFull = MODE != kDiluFactor && HMASK == 0;
+    constexpr bool kCanFull = MODE != kDiluFactor;
     const size_t recBytes = (size_t)nSteps * G * 64 * sizeof(R);
-    const bool fullWave = kCanFull && !delivers && recBytes <= (size_t)INT_MAX;
+    const bool fullWave = kCanFull && recBytes <= (size_t)INT_MAX;
     const auto rRec = rawBuffer(recs + (size_t)s0 * G * 64, fullWave ? recBytes : 0);
-    const auto rCode = rawBuffer(codes + (size_t)s0 * H * 64, fullWave ? (size_t)nSteps * H * 64 * sizeof(int4) : 0);
+    const auto rCode = rawBuffer(codes + (size_t)s0 * NC * 64, fullWave ? (size_t)nSteps * NC * 64 * sizeof(int) : 0);
     const auto rIn = rawBuffer(kCanFull ? in + (size_t)s0 * 64 : nullptr, fullWave ? (size_t)nSteps * 64 * sizeof(T) : 0);
     const auto rOut = rawBuffer(kCanFull ? out + (size_t)s0 * 64 : nullptr, fullWave ? (size_t)nSteps * 64 * sizeof(T) : 0);
-    const unsigned vRec = lane * (unsigned)sizeof(R), vCode = lane * (unsigned)sizeof(int4),
+    const unsigned vRec = lane * (unsigned)sizeof(R), vCode = lane * (unsigned)sizeof(int),
                    vRow = lane * (unsigned)sizeof(T);
     auto loadF = [&](int i, Step &S) {
         const unsigned j = (unsigned)(MODE == kDiluBwd ? nSteps - 1 - i : i);
 #pragma unroll
         for (int g = 0; g < G; ++g) S.v[g] = bufLoad<R, 0>(rRec, vRec + g * 64 * sizeof(R), j * G * 64 * sizeof(R));
 #pragma unroll
-        for (int h = 0; h < H; ++h) S.c[h] = bufLoad<int4, 0>(rCode, vCode + h * 64 * sizeof(int4), j * H * 64 * sizeof(int4));
+        for (int h = 0; h < NC; ++h) S.c[h] = bufLoad<int, 0>(rCode, vCode + h * 64 * sizeof(int), j * NC * 64 * sizeof(int));
         S.a = bufLoad<T, 0>(rIn, vRow, j * 64 * sizeof(T));
     };
 
     if (active && nSteps > 0) {
         // ring slots above the wave's kRing steps hold zeros: a code without
-        // a ring slot (kCodeInbox, kCodeNone) reads a finite zero there
+        // a ring slot (kCodeNone) reads a finite zero there
         for (int q = kRing * 64 + lane; q < kRingSlots; q += 64) ring[q] = T(0);
         __builtin_amdgcn_wave_barrier();
         Step buf[kPrefetch];
@@ -151,9 +116,7 @@ __global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState 
         // back, and the slot the step overwrites is never among them), so the
         // LDS round trip overlaps the rest of the previous step.  The code
         // byte is the ring slot.
-        auto ringSlot = [&](const Step &S, int k) {
-            return (elem(S.c[k / 16], (k / 4) % 4) >> (8 * (k % 4))) & 0xFF;
-        };
+        auto ringSlot = [&](const Step &S, int k) { return (S.c[k / 4] >> (8 * (k % 4))) & 0xFF; };
         T rv[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) rv[k] = ring[ringSlot(buf[0], k)];
@@ -164,12 +127,12 @@ __global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState 
         // number of ring rounds, so every step's ring slot is a constant.
         //
         // A group is FULL when its steps and their prefetches all lie inside
-        // the wave's steps, in a sweep without inbox values or deliveries:
-        // there nothing is clamped, the store is unconditional, every address
-        // is a scalar offset plus a lane constant, and each dependency term is
-        // taken without a select (a missing dependency has a zero coefficient
-        // and reads a zero slot, so for rD >= 0 its term is +0 and leaves the
-        // value unchanged bit for bit).
+        // the wave's steps: there nothing is clamped, the store is
+        // unconditional, every address is a scalar offset plus a lane
+        // constant, and each dependency term is taken without a select (a
+        // missing dependency has a zero coefficient and reads a zero slot, so
+        // for rD >= 0 its term is +0 and leaves the value unchanged bit for
+        // bit).
         auto runGroup = [&](int i0, auto fullTag) {
             constexpr bool FULL = decltype(fullTag)::value;
 #pragma unroll
@@ -178,64 +141,21 @@ __global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState 
                 const int i = i0 + uu;
                 const bool inRange = FULL || i < nSteps;
                 Step &S = buf[u];
-                const int s = FULL ? 0 : sliceOf(i);
-                int code[K];
-                T c[K];
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    code[k] = (elem(S.c[k / 16], (k / 4) % 4) >> (8 * (k % 4))) & 0xFF;
-                    c[k] = (T)elem(S.v[k / N], k % N);
-                }
                 const T last = (T)elem(S.v[K / N], K % N);   // rD, or diag for the factor
-                // rare slow path (wave-uniform branch): an inbox value not yet
-                // delivered when it was prefetched is polled here, and the
-                // inbox prefetches of the following steps are refreshed so
-                // that one late producer costs one wait, not one per step
-                if constexpr (!FULL && KI > 0) {
-                    bool miss = false;
-#pragma unroll
-                    for (int k = 0; k < K; ++k)
-                        if (HMASK & (1 << k))
-                            miss |= inRange && code[k] == kCodeInbox &&
-                                    S.hv[__builtin_popcount(HMASK & ((1 << k) - 1))] == kSent;
-                    if (__builtin_expect(__any(miss), 0)) {
-                        ++nSlow;
-#pragma unroll
-                        for (int k = 0; k < K; ++k)
-                            if (HMASK & (1 << k)) {
-                                const int kk = __builtin_popcount(HMASK & ((1 << k) - 1));
-                                if (code[k] == kCodeInbox && S.hv[kk] == kSent)
-                                    S.hv[kk] = haloWait(inbox, ((s * KI + kk) << 6) + lane, kSent, V.err);
-                            }
-#pragma unroll
-                        for (int d = 1; d < kPrefetch; ++d) {
-                            Step &F = buf[(u + d) % kPrefetch];
-                            const int sf = sliceOf(i + d);
-#pragma unroll
-                            for (int kk = 0; kk < KI; ++kk)
-                                if (F.hv[kk] == kSent) F.hv[kk] = haloLoad(inbox, ((sf * KI + kk) << 6) + lane);
-                        }
-                        __builtin_amdgcn_s_waitcnt(0);
-                    }
-                }
-                // branch-free: ring or inbox value per dependency; a missing
-                // dependency contributes an exact zero
+                // branch-free: a missing dependency contributes an exact zero
                 T y;
                 if (MODE == kDiluFwd) y = S.a * last;
                 else if (MODE == kDiluBwd) y = S.a;
                 else y = last;
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
-                    T v = rv[k];
-                    if (HMASK & (1 << k)) {
-                        const U h = S.hv[__builtin_popcount(HMASK & ((1 << k) - 1))];
-                        v = code[k] == kCodeInbox ? Bits<T>::from(h) : v;
-                    }
-                    const bool has = code[k] != kCodeNone;
-                    if (MODE == kDiluFactor) y = has ? y - c[k] / v : y;
-                    else if (FULL) y = y - last * c[k] * v;
-                    else y = has ? y - last * c[k] * v : y;
+                    const T c = (T)elem(S.v[k / N], k % N);
+                    const bool has = ringSlot(S, k) != kCodeNone;
+                    if (MODE == kDiluFactor) y = has ? y - c / rv[k] : y;
+                    else if (FULL) y = y - last * c * rv[k];
+                    else y = has ? y - last * c * rv[k] : y;
                 }
+                const int s = FULL ? 0 : sliceOf(i);
                 // the ring is private to this wavefront and LDS operations of
                 // a wavefront execute in order: no barrier (which would also
                 // drain the prefetch loads) is needed between steps
@@ -260,16 +180,6 @@ __global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState 
                     } else {
                         out[p] = y;
                     }
-                    // deliver the value to the inboxes of its consumers in other waves
-                    if (delivers) {
-#pragma unroll
-                        for (int j = 0; j < K; ++j) {
-                            const int o = elem(S.c[(NC + j) / 4], (NC + j) % 4);
-                            if (o >= 0)
-                                __hip_atomic_store(&inbox[o], Bits<T>::to(y), __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-                        }
-                    }
                 }
                 load(i + kPrefetch, S);
             }
@@ -283,12 +193,137 @@ __global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState 
         unsigned long long *tr = V.trace + 4 * (size_t)blockIdx.x;
         tr[0] = tStart;
         tr[1] = wall_clock64();
-        tr[2] = nSlow;
+        tr[2] = 0;
         tr[3] = (unsigned long long)nSteps;
     }
-    // reset the inbox of the next sweep (nobody reads it during this one)
-    if (inboxClear)
-        for (int q = blockIdx.x * 64 + lane; q < nClear; q += gridDim.x * 64) inboxClear[q] = kSent;
+}
+
+// A level group: one workgroup sweeps a whole region, level by level, up to 16
+// slices of a level at a time (one per wave), with a barrier after each level.
+// A row's dependencies come from an LDS ring of the region's last kLevelRing
+// rows (which spans tens of levels of a mesh of 10^5 cells), or from memory if
+// they lie further back.  Rows are loaded kDeep rounds ahead.
+//
+// The alternative, a wave per 64 rows of a level with every dependency passed
+// through memory, costs a memory round trip per level and floods the fabric
+// with the polls of waves whose turn is far off: 1257 us a sweep on 78k cells
+// renumbered along a front (122 levels of up to 957 rows), against what is
+// bound here by one CU's load path (60 bytes a row in FP64, about 64 bytes a
+// clock) and the barrier.  Two regions of a system, or the systems of a batch,
+// run side by side on CUs of their own.
+template <int K>
+constexpr int kDeepOf = K <= 3 ? 3 : K <= 6 ? 2 : 1;
+
+template <typename T, int K, int MODE>
+__global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysState *st, const T *in, T *out)
+{
+    using R = typename RecordOf<T, MODE>::V;
+    constexpr int N = RecordOf<T, MODE>::N;
+    constexpr int G = packChunks(K + 1, N);
+    constexpr int kDeep = kDeepOf<K>;
+    __shared__ T ring[kLevelRing];
+    const LevelGroup g = V.groups[blockIdx.x];
+    if (MODE != kDiluFactor && st[g.sys].status != kRunning) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned long long tStart = V.trace ? wall_clock64() : 0ull;
+    const int2 *rounds = V.lvRounds + g.round0;
+    const int32_t *deps = MODE == kDiluBwd ? V.bDeps : V.fDeps;
+    const R *recs = MODE == kDiluFactor ? (const R *)V.prodPack : (const R *)(MODE == kDiluBwd ? V.bPack : V.fPack);
+    // what a later row reads back when it is out of the ring (the factor: d)
+    const T *back = MODE == kDiluFactor ? nullptr : out + (size_t)g.slice0 * 64;
+
+    struct Item {
+        R v[G];
+        int c[K];
+        T a;
+        int s;       // the wave's slice, -1: none in this round
+        int flags;
+    };
+    auto load = [&](int i, Item &S) {
+        int2 r = rounds[MODE == kDiluBwd ? g.nRounds - 1 - min(i, g.nRounds - 1) : min(i, g.nRounds - 1)];
+        const bool has = i < g.nRounds && wave < (r.y >> 2);
+        const int s = r.x + (has ? wave : 0);   // (a slice to load from in any case: no load is conditional)
+#pragma unroll
+        for (int q = 0; q < G; ++q) S.v[q] = recs[((size_t)s * G + q) * 64 + lane];
+#pragma unroll
+        for (int k = 0; k < K; ++k) S.c[k] = deps[((size_t)s * K + k) * 64 + lane];
+        if (MODE != kDiluFactor) S.a = in[(size_t)s * 64 + lane];
+        S.s = has ? s : -1;
+        S.flags = r.y & 3;
+    };
+    Item buf[kDeep];
+#pragma unroll
+    for (int u = 0; u < kDeep; ++u) load(u, buf[u]);
+    for (int i0 = 0; i0 < g.nRounds; i0 += kDeep) {
+#pragma unroll
+        for (int u = 0; u < kDeep; ++u) {
+            const int i = i0 + u;
+            Item &S = buf[u];
+            if (i < g.nRounds && S.s >= 0) {
+                const T last = (T)elem(S.v[K / N], K % N);   // rD, or diag for the factor
+                T v[K];
+                bool far = false;
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    far |= S.c[k] >= kLevelRing;
+                    v[k] = ring[S.c[k] & (kLevelRing - 1)];
+                }
+                if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
+                    // (stored more than kDeep rounds ago by a wave of this
+                    // workgroup, which has waited since for loads issued
+                    // after that store: it has reached the CU's cache; the
+                    // factor reads the 1/d it stored, hence d's own copy)
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (S.c[k] >= kLevelRing) v[k] = MODE == kDiluFactor ? (T)V.lvD[(size_t)g.slice0 * 64 + S.c[k] - kLevelRing] : back[S.c[k] - kLevelRing];
+                }
+                T y;
+                if (MODE == kDiluFwd) y = S.a * last;
+                else if (MODE == kDiluBwd) y = S.a;
+                else y = last;
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const T c = (T)elem(S.v[k / N], k % N);
+                    const bool has = S.c[k] != kNoDep;
+                    if (MODE == kDiluFactor) y = has ? y - c / v[k] : y;
+                    else y = has ? y - last * c * v[k] : y;
+                }
+                const size_t p = (size_t)S.s * 64 + lane;
+                ring[(p - (size_t)g.slice0 * 64) & (kLevelRing - 1)] = y;
+                if (MODE == kDiluFactor) {
+                    const double rd = V.cellOfPos[p] >= 0 ? 1.0 / (double)y : 0.0;
+                    V.rDout[p] = rd;
+                    V.lvD[p] = (double)y;
+                    constexpr int NP = Pack<double>::N;
+                    constexpr int GP = packChunks(K + 1, NP);
+                    ((double *)&V.fPack[((size_t)S.s * GP + K / NP) * 64 + lane])[K % NP] = rd;
+                    ((double *)&V.bPack[((size_t)S.s * GP + K / NP) * 64 + lane])[K % NP] = rd;
+                } else {
+                    out[p] = y;
+                }
+            }
+            const bool ends = i < g.nRounds && (S.flags & (MODE == kDiluBwd ? kRoundFirst : kRoundLast));
+            load(i + kDeep, S);
+            if (ends) {
+                // the level's values are in the ring before any wave goes on.
+                // (Only LDS is waited for: a full fence would drain the rows
+                // in flight.  Values further back than the ring may be as
+                // recent as the last level only where levels are wider than
+                // a quarter of it: there the stores are waited for too.)
+                if (V.lvDrain) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            }
+        }
+    }
+    if (V.trace && threadIdx.x == 0) {
+        unsigned long long *tr = V.trace + 4 * ((size_t)V.nWaves + V.nBoxWaves + blockIdx.x);
+        tr[0] = tStart;
+        tr[1] = wall_clock64();
+        tr[2] = 0;
+        tr[3] = (unsigned long long)g.nRounds;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -493,21 +528,22 @@ __global__ void k_convert_rd(DiluView<float> V, const double *rD64, int nPos)
 // Launchers
 // ---------------------------------------------------------------------------
 
-template <typename T, int MODE>
-static hipError_t launchK(const DiluView<T> &V, const SysState *st, const T *in, T *out,
-                          typename Bits<T>::U *use, typename Bits<T>::U *clr, int nClr, hipStream_t s)
+template <typename T, int K, int MODE>
+static void launchGeneralK(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s)
 {
-    if (V.nWaves <= 0) return hipSuccess;
-    if (!V.waveOut) return hipErrorInvalidValue;
-    const int mask = effectiveHaloMask(V.K, MODE == kDiluBwd ? V.haloMaskB : V.haloMaskF);
+    if (V.nWaves > 0) k_dilu_wave<T, K, MODE><<<V.nWaves, 64, 0, s>>>(V, st, in, out);
+    if (V.nGroups > 0) k_dilu_levels<T, K, MODE><<<V.nGroups, 64 * V.lvWaves, 0, s>>>(V, st, in, out);
+}
+
+template <typename T, int MODE>
+static hipError_t launchGeneral(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s)
+{
+    if (V.nWaves <= 0 && V.nGroups <= 0) return hipSuccess;
+    if (V.lvWaves < 1 || V.lvWaves > 16) return hipErrorInvalidValue;
     switch (V.K) {
-    case 3:
-        if (mask == 0) k_dilu_wave<T, 3, MODE, 0><<<V.nWaves, 64, 0, s>>>(V, st, in, out, use, clr, nClr);
-        else if (mask == 3) k_dilu_wave<T, 3, MODE, 3><<<V.nWaves, 64, 0, s>>>(V, st, in, out, use, clr, nClr);
-        else k_dilu_wave<T, 3, MODE, 7><<<V.nWaves, 64, 0, s>>>(V, st, in, out, use, clr, nClr);
-        break;
-    case 6: k_dilu_wave<T, 6, MODE, 63><<<V.nWaves, 64, 0, s>>>(V, st, in, out, use, clr, nClr); break;
-    case 12: k_dilu_wave<T, 12, MODE, 4095><<<V.nWaves, 64, 0, s>>>(V, st, in, out, use, clr, nClr); break;
+    case 3: launchGeneralK<T, 3, MODE>(V, st, in, out, s); break;
+    case 6: launchGeneralK<T, 6, MODE>(V, st, in, out, s); break;
+    case 12: launchGeneralK<T, 12, MODE>(V, st, in, out, s); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -535,7 +571,7 @@ static hipError_t launchBoxFactor(const DiluView<double> &V, hipStream_t s)
 template <typename T, typename GenF, typename BoxF>
 static hipError_t bothSweeps(const DiluView<T> &V, hipStream_t s, GenF &&gen, BoxF &&box)
 {
-    const bool fork = V.side && V.fork && V.join && V.nWaves > 0 && V.nBoxWaves > 0;
+    const bool fork = V.side && V.fork && V.join && V.nWaves + V.nGroups > 0 && V.nBoxWaves > 0;
     if (!fork) {
         hipError_t e = gen(s);
         return e != hipSuccess ? e : box(s);
@@ -552,21 +588,16 @@ static hipError_t bothSweeps(const DiluView<T> &V, hipStream_t s, GenF &&gen, Bo
 template <typename T>
 hipError_t diluForward(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s)
 {
-    using U = typename Bits<T>::U;
     return bothSweeps(
-        V, s, [&](hipStream_t q) { return launchK<T, kDiluFwd>(V, st, in, out, (U *)V.haloF, (U *)V.haloB, V.nHaloB, q); },
+        V, s, [&](hipStream_t q) { return launchGeneral<T, kDiluFwd>(V, st, in, out, q); },
         [&](hipStream_t q) { return boxForward<T>(V, st, in, out, q); });
 }
 
 template <typename T>
 hipError_t diluBackward(const DiluView<T> &V, const SysState *st, T *inout, hipStream_t s)
 {
-    using U = typename Bits<T>::U;
     return bothSweeps(
-        V, s,
-        [&](hipStream_t q) {
-            return launchK<T, kDiluBwd>(V, st, inout, inout, (U *)V.haloB, (U *)V.haloF, V.nHaloF, q);
-        },
+        V, s, [&](hipStream_t q) { return launchGeneral<T, kDiluBwd>(V, st, inout, inout, q); },
         [&](hipStream_t q) { return boxBackward<T>(V, st, inout, q); });
 }
 
@@ -582,13 +613,10 @@ __global__ void k_fill_u32(unsigned int *a, int n, unsigned int v)
 
 hipError_t diluFactor(const DiluView<double> &V, hipStream_t s)
 {
-    // the factor publishes d through its own inbox buffer, reset first
-    const int n = V.nHaloF + V.nBoxIn;
-    k_fill_u64<<<256, 256, 0, s>>>((unsigned long long *)V.haloC, n > 0 ? n : 1, kHaloSentinel64);
-    hipError_t e = launchK<double, kDiluFactor>(V, nullptr, nullptr, nullptr, (unsigned long long *)V.haloC,
-                                                nullptr, 0, s);
-    if (e != hipSuccess) return e;
-    return launchBoxFactor(V, s);
+    // box tiles publish d through an inbox buffer of their own, reset first
+    if (V.nBoxIn > 0) k_fill_u64<<<256, 256, 0, s>>>((unsigned long long *)V.boxInC, V.nBoxIn, kHaloSentinel64);
+    hipError_t e = launchGeneral<double, kDiluFactor>(V, nullptr, nullptr, nullptr, s);
+    return e != hipSuccess ? e : launchBoxFactor(V, s);
 }
 
 hipError_t diluFactorTileLocal(const DiluView<double> &V, double *rD, int segs, hipStream_t s)

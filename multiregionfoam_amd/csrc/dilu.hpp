@@ -12,7 +12,7 @@ namespace mrfg {
 
 enum { kDiluFwd = 0, kDiluBwd = 1, kDiluFactor = 2 };
 
-// Halo slots hold the raw bits of a value; a slot equal to the sentinel has
+// Inbox entries of box tiles hold the raw bits of a value; one equal to the sentinel has
 // not been published yet in the current sweep (signalling-NaN payloads that
 // arithmetic never produces).
 constexpr unsigned long long kHaloSentinel64 = 0xFFF4A5A5A5A5A5A5ull;
@@ -24,12 +24,12 @@ constexpr unsigned int kHaloSentinel32 = 0xFFA5A5A5u;
 //   values  [c_0..c_{K-1}, rD]: forward = lower coefficients, backward =
 //           upper coefficients, factor = upper*lower products with the
 //           diagonal in place of rD;
-//   ints    [codes, out_0..out_{K-1}]: one byte per dependency (kCodeNone,
-//           kCodeInbox, or an LDS ring slot 0..255), four per int, then the
-//           inbox addresses this row's value is delivered to (-1: none).
-// A dependency on another wave is read from the consumer's inbox slot
-// (slice, kk, lane), kk = rank of the dependency slot among the slots that
-// can cross waves, so its prefetch needs no other load first.
+// Rows of general waves also have codes that say where each dependency is:
+//   chains        one byte each (kCodeNone or an LDS ring slot), four per
+//                 int, int j of lane l of slice s at (s*NC + j)*64 + l;
+//   level groups  one int each, that of slot k at (s*K + k)*64 + l: kNoDep,
+//                 an LDS ring slot (< kLevelRing), or kLevelRing + the row's
+//                 place in the group.
 template <typename T>
 struct Pack;
 template <>
@@ -43,32 +43,33 @@ struct Pack<float> {
     static constexpr int N = 4;
 };
 constexpr int packChunks(int n, int per) { return (n + per - 1) / per; }
-constexpr int kCodeNone = 0xFF, kCodeInbox = 0xFE;
-// ints per row: packed codes then K outs
-constexpr int codeInts(int K) { return packChunks(K, 4) + K; }
-// Dependency slots that are given an inbox for a K-slot schedule whose
-// cross-wave dependencies occur in `mask`: structured-box schedules (K = 3)
-// only cross waves in the first two slots; anything else gets all slots.
-inline int effectiveHaloMask(int K, int mask)
-{
-    if (K == 3 && mask == 0) return 0;   // no cross-wave dependency: no inbox at all
-    return (K == 3 && (mask & ~3) == 0) ? 3 : (1 << K) - 1;
-}
+constexpr int kCodeNone = 0xFF;
+
+// One workgroup's sweep of a level group: rounds of up to lvWaves slices, the
+// first slice and (count << 2 | flags) of each in `lvRounds`
+enum { kRoundLast = 1, kRoundFirst = 2 };   // the round ends / starts a level
+struct LevelGroup {
+    int slice0, round0, nRounds, sys;
+};
 
 template <typename T>
 struct DiluView {
-    const int32_t *order = nullptr;      // general (code-driven) waves in forward dispatch order
+    // chain waves in dispatch order
+    const int32_t *order = nullptr;
     const int32_t *waveSlice = nullptr, *waveSteps = nullptr, *waveSys = nullptr;
     int nWaves = 0, K = 3;
-    const int4 *fCodes = nullptr, *bCodes = nullptr;
-    const int32_t *waveOut = nullptr;    // per wave: bit 0 / 1 when it delivers forward / backward values
+    const int32_t *fCodes = nullptr, *bCodes = nullptr;
+    // level groups
+    const LevelGroup *groups = nullptr;
+    const int2 *lvRounds = nullptr;
+    const int32_t *fDeps = nullptr, *bDeps = nullptr;
+    int nGroups = 0, lvWaves = 1;
+    bool lvDrain = false;                // a level is wider than a quarter of the ring
+    double *lvD = nullptr;               // factor: d per row of the level groups
     typename Pack<T>::V *fPack = nullptr, *bPack = nullptr;
     const double2 *prodPack = nullptr;   // factor records (FP64)
     double *rDout = nullptr;             // factor: plain rD per row
     const int32_t *cellOfPos = nullptr;  // factor: padding rows get rD = 0
-    int haloMaskF = 0, haloMaskB = 0;    // dependency slots that may cross waves
-    void *haloF = nullptr, *haloB = nullptr, *haloC = nullptr;   // inboxes
-    int nHaloF = 0, nHaloB = 0;          // inbox sizes (values)
     int *err = nullptr;                  // bit 2: a halo wait expired
     // structured-box tiles (dilu_box.hip; the factor in dilu.hip): their own
     // dispatch order, kBoxMeta ints of tile geometry per wave, and compact
@@ -86,8 +87,8 @@ struct DiluView {
     void *boxInF = nullptr, *boxInB = nullptr, *boxInC = nullptr;
     int nBoxIn = 0;
     // optional trace: per wave start / end realtime clock ticks, slow-path
-    // hits and steps (4 entries each); general waves by dispatch index, then
-    // box waves by dispatch index
+    // hits and steps (4 entries each); chain waves by dispatch index, then box
+    // tiles, then level groups
     unsigned long long *trace = nullptr;
     // host side: when both kinds of waves exist, the box sweep runs on `side`
     // concurrently with the general sweep (regions never depend on each
@@ -136,7 +137,7 @@ hipError_t diluApplyFused(const DiluView<T> &V, const SysState *st, int inp, con
 template <typename T>
 bool diluCanFuse(const DiluView<T> &V)
 {
-    return V.nWaves == 0 && V.nBoxWaves > 0 && V.K == 3;
+    return V.nWaves == 0 && V.nGroups == 0 && V.nBoxWaves > 0 && V.K == 3;
 }
 // Factorisation: rD = 1/d for every row of the batch (FP64), written to
 // rDout and into the forward and backward records.

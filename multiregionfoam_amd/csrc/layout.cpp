@@ -23,6 +23,7 @@ struct WaveBuild {
     // structured-box tile (box = false for level waves)
     bool box = false;
     int tb = 0, tc = 0, TB = 0, nA = 0, seqAxis = 0, actB = 0, actC = 0;
+    std::vector<int32_t> levels;   // level group: slices per level
 };
 
 void tangential(int a, int &b, int &c)
@@ -121,37 +122,29 @@ void levelWaves(int regionIdx, int c0, int c1, const RowDeps &D, RegionSchedule 
     for (int c = c0; c < c1; ++c) byLevel[level[c - c0]].push_back(c);
     size_t maxWidth = 0;
     for (const auto &b : byLevel) maxWidth = std::max(maxWidth, b.size());
-    if (maxWidth <= (size_t)kSlice) {
-        // every level fits one slice (e.g. 2-D and multi-block meshes whose
-        // levels are anti-diagonals of at most 64 cells): one wave walks the
-        // levels as its steps, so a dependency on the previous levels comes
-        // from the wave's own LDS ring instead of another wave's inbox
-        rs.kind = "chain";
-        WaveBuild w;
-        w.key = 0;
-        w.region = regionIdx;
-        w.steps = maxLevel + 1;
-        w.cells.assign((size_t)w.steps * kSlice, -1);
-        for (int lv = 0; lv <= maxLevel; ++lv)
-            for (size_t l = 0; l < byLevel[lv].size(); ++l) w.cells[(size_t)lv * kSlice + l] = byLevel[lv][l];
-        out.push_back(std::move(w));
-        rs.nWaves++;
-        rs.maxSteps = maxLevel + 1;
-        return;
+    int reach = 1;   // levels between a cell and its furthest neighbour
+    for (int c = c0; c < c1; ++c)
+        for (int q = D.lo_off[c]; q < D.lo_off[c + 1]; ++q) reach = std::max(reach, level[c - c0] - level[D.lo_nb[q] - c0]);
+    WaveBuild w;
+    w.key = 0;
+    w.region = regionIdx;
+    // one wave walks narrow levels as its steps: every dependency comes from
+    // its own LDS ring and no step waits for another wave.  Wider levels (or
+    // levels that reach further back) go to a workgroup with a barrier per
+    // level.
+    const bool chain = maxWidth <= (size_t)kSlice && reach <= kRing - 1;
+    for (int lv = 0; lv <= maxLevel; ++lv) {
+        const int n = (int)((byLevel[lv].size() + kSlice - 1) / kSlice);
+        const size_t at = w.cells.size();
+        w.cells.resize(at + (size_t)n * kSlice, -1);
+        std::copy(byLevel[lv].begin(), byLevel[lv].end(), w.cells.begin() + at);
+        if (!chain) w.levels.push_back(n);
+        w.steps += n;
     }
-    rs.kind = "levels";
-    for (int lv = 0; lv <= maxLevel; ++lv)
-        for (size_t i = 0; i < byLevel[lv].size(); i += kSlice) {
-            WaveBuild w;
-            w.key = lv;
-            w.region = regionIdx;
-            w.steps = 1;
-            w.cells.assign(kSlice, -1);
-            for (size_t l = 0; l < (size_t)kSlice && i + l < byLevel[lv].size(); ++l) w.cells[l] = byLevel[lv][i + l];
-            out.push_back(std::move(w));
-            rs.nWaves++;
-        }
-    rs.maxSteps = 1;
+    rs.kind = chain ? "chain" : "levels";
+    rs.nWaves = 1;
+    rs.maxSteps = w.steps;
+    out.push_back(std::move(w));
 }
 
 }  // namespace
@@ -260,12 +253,14 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
     L.waveSlice.resize(L.nWaves);
     L.waveSteps.resize(L.nWaves);
     L.waveKey.resize(L.nWaves);
+    L.waveLevels.resize(L.nWaves);
     int slice = 0;
     for (int wi = 0; wi < L.nWaves; ++wi) {
         const WaveBuild &w = waves[ord[wi]];
         L.waveSlice[wi] = slice;
         L.waveSteps[wi] = w.steps;
         L.waveKey[wi] = w.key;
+        L.waveLevels[wi] = w.levels;
         slice += w.steps;
     }
     L.nSlices = slice;
@@ -288,6 +283,19 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
     }
     for (int c = 0; c < N; ++c)
         if (L.posOfCell[c] < 0) throw std::runtime_error("DILU schedule does not cover every cell");
+
+    // level groups: first and one-past-last slice (of the wave) of each slice's level
+    std::vector<int32_t> lvBegin(L.nSlices, -1), lvEnd(L.nSlices, -1);
+    for (int wi = 0; wi < L.nWaves; ++wi) {
+        int t = 0;
+        for (int n : L.waveLevels[wi]) {
+            for (int k = 0; k < n; ++k) {
+                lvBegin[L.waveSlice[wi] + t + k] = t;
+                lvEnd[L.waveSlice[wi] + t + k] = t + n;
+            }
+            t += n;
+        }
+    }
 
     // structured-box waves: tile neighbours and fixed-slot records (slot =
     // 2 - axis: z, y, x, the face order of a cell's lower neighbours and the
@@ -419,8 +427,6 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
     L.bVal.assign(nDep, 0.0);
     L.fSrc.assign(nDep, -1);
     L.bSrc.assign(nDep, -1);
-    L.fHalo.assign(L.nPos, -1);
-    L.bHalo.assign(L.nPos, -1);
 
     auto waveStep = [&](int p, int &w, int &t, int &lane) {
         int s = p / kSlice;
@@ -494,13 +500,15 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
                     L.fVal[e] = lo[f];
                     L.fProd[e] = R.upper[f] * lo[f];
                     L.fSrc[e] = loSrc(f);
-                    if (wd == w && t - td >= 1 && t - td <= kRing - 1) {
-                        L.fCode[e] = -((td % kRing) * kSlice + ld + 1);
+                    if (wd != w) throw std::runtime_error("DILU dependency crosses waves");
+                    if (lvEnd[s] >= 0) {
+                        if (lvEnd[pd / kSlice] > lvBegin[s]) throw std::runtime_error("DILU schedule violates a forward dependency");
+                        // in the ring until the rows kLevelRing further on are written
+                        const int at = td * kSlice + ld;
+                        L.fCode[e] = lvEnd[s] * kSlice - at <= kLevelRing ? at & (kLevelRing - 1) : kLevelRing + at;
                     } else {
-                        if (wd == w ? td >= t : wd > w)
-                            throw std::runtime_error("DILU schedule violates a forward dependency");
-                        if (L.fHalo[pd] < 0) L.fHalo[pd] = L.nHaloF++;
-                        L.fCode[e] = L.fHalo[pd];
+                        if (t - td < 1 || t - td > kRing - 1) throw std::runtime_error("DILU schedule violates a forward dependency");
+                        L.fCode[e] = (td % kRing) * kSlice + ld;
                     }
                 }
                 // backward sweep: upper neighbours, reverse face order; processing
@@ -513,14 +521,14 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
                     size_t e = ((size_t)s * K + k) * kSlice + l;
                     L.bVal[e] = R.upper[D.up_face[q]];
                     L.bSrc[e] = upSrc(D.up_face[q]);
-                    if (wd == w && td - t >= 1 && td - t <= kRing - 1) {
-                        int id = T - 1 - td;
-                        L.bCode[e] = -((id % kRing) * kSlice + ld + 1);
+                    if (wd != w) throw std::runtime_error("DILU dependency crosses waves");
+                    if (lvEnd[s] >= 0) {
+                        if (lvBegin[pd / kSlice] < lvEnd[s]) throw std::runtime_error("DILU schedule violates a backward dependency");
+                        const int at = td * kSlice + ld;
+                        L.bCode[e] = at - lvBegin[s] * kSlice < kLevelRing ? at & (kLevelRing - 1) : kLevelRing + at;
                     } else {
-                        if (wd == w ? td <= t : wd < w)
-                            throw std::runtime_error("DILU schedule violates a backward dependency");
-                        if (L.bHalo[pd] < 0) L.bHalo[pd] = L.nHaloB++;
-                        L.bCode[e] = L.bHalo[pd];
+                        if (td - t < 1 || td - t > kRing - 1) throw std::runtime_error("DILU schedule violates a backward dependency");
+                        L.bCode[e] = ((T - 1 - td) % kRing) * kSlice + ld;
                     }
                 }
             }

@@ -11,13 +11,18 @@
 //     with a skew of b+c steps, so each of a cell's three lower neighbours
 //     was computed one step earlier by the same or an adjacent lane;
 //   * any other region is scheduled by levels (a cell's level is one more
-//     than its lower neighbours' largest), 64 rows of one level per wave.
+//     than its lower neighbours' largest): a chain, one wave whose steps are
+//     the levels, where every level fits 64 rows and reaches at most
+//     kRing - 1 levels back (2-D and multi-block meshes, whose levels are
+//     anti-diagonals), else a level group, swept by one workgroup that meets
+//     at a barrier after each level.
 //
 // Either way the schedule is a topological order of the factor's dependency
 // graph, so the Cholesky/DILU factor and sweeps computed in it are the
-// reference preconditioner itself.  A dependency on a row of the same wave
-// at most kRing-1 steps back is read from the wave's LDS ring; any other is
-// read from a halo slot the producing wave publishes.
+// reference preconditioner itself.  A chain's wave reads its dependencies
+// from an LDS ring of its last kRing steps, a level group from an LDS ring of
+// the region's last kLevelRing rows, or from memory where they lie further
+// back.
 //
 // Per slice of 64 rows:
 //   SpMV   sliced ELL, column-major inside the slice: entry k of lane l at
@@ -29,7 +34,9 @@
 //   DILU   K dependency slots per row at (s*K + k)*64 + l: forward = lower
 //          neighbours in face order with lower coefficients and upper*lower
 //          products, backward = upper neighbours in reverse face order with
-//          upper coefficients; codes: kNoDep, ring slot -(slot+1), or halo.
+//          upper coefficients; codes: kNoDep, in a chain the ring slot, in a
+//          level group the ring slot or kLevelRing + the row's place in the
+//          region's slices.
 #pragma once
 
 #include "coupled_system.hpp"
@@ -44,7 +51,8 @@ namespace mrfg {
 constexpr int kSlice = 64;          // rows per slice = wavefront size
 constexpr int kSlicesPerBlock = 4;  // 256-thread blocks for SpMV / vector ops
 constexpr int kRing = 3;            // LDS ring depth (steps) of a DILU wave (slots < 192)
-constexpr int32_t kNoDep = INT32_MIN;
+constexpr int32_t kNoDep = -1;
+constexpr int kLevelRing = 16384;   // rows of a level group's LDS ring (128 KB in FP64); a power of two
 
 // Per-wave metadata of a structured-box tile wave (kBoxMeta ints each).
 enum {
@@ -65,7 +73,7 @@ enum {
 };
 
 struct RegionSchedule {
-    std::string kind;                // "box" or "levels"
+    std::string kind;                // "box", "chain" or "levels"
     int n[3] = {0, 0, 0};            // box dimensions
     int seqAxis = -1, tileB = 0, tileC = 0;
     int nWaves = 0, maxSteps = 0;
@@ -96,8 +104,8 @@ struct SystemLayout {
     // DILU
     std::vector<int32_t> fCode, bCode;       // nSlices * K * 64
     std::vector<double> fVal, fProd, bVal;
-    std::vector<int32_t> fHalo, bHalo;       // per position: halo slot published or -1
-    int nHaloF = 0, nHaloB = 0;
+    // per wave: the slices of each level of a level group (empty for others)
+    std::vector<std::vector<int32_t>> waveLevels;
     // structured-box tile waves: their rows keep the DILU values in fixed
     // slots (slot = 2 - axis of the neighbour: z, y, x, which is both the
     // face order of the lower neighbours and the reverse face order of the
