@@ -133,6 +133,21 @@ struct Tile {
     __device__ int cell(int b, int c) const { return FWD ? (c + 1) * (TB + 1) + b + 1 : c * (TB + 1) + b; }
 };
 
+// the value of lane l - 1 (forward) / l + 1 (backward), zero past the wave's end
+template <typename T, bool FWD>
+__device__ inline T laneBefore(T v)
+{
+    auto move = [](unsigned u) {   // wave_shr:1 / wave_shl:1
+        return (unsigned)__builtin_amdgcn_update_dpp(0, (int)u, FWD ? 0x138 : 0x130, 0xf, 0xf, true);
+    };
+    if constexpr (sizeof(T) == 8) {
+        const unsigned long long u = Bits<T>::to(v);
+        return Bits<T>::from(((unsigned long long)move((unsigned)(u >> 32)) << 32) | move((unsigned)u));
+    } else {
+        return Bits<T>::from(move(Bits<T>::to(v)));
+    }
+}
+
 // The rows [lo, hi) of the sequential axis that a workgroup sweeps
 struct Span {
     int lo, hi;
@@ -143,7 +158,8 @@ struct Span {
 // ---------------------------------------------------------------------------
 
 // FLAT: the tile has no neighbour along c at all (one line of cells across,
-// as in 2-D): the c term is left out.
+// as in 2-D): the c term is left out, and a LONE tile needs no plane, since
+// the one exchange left is a DPP move.
 template <typename T, int MODE, int AX, bool LONE, bool FLAT>
 __device__ __forceinline__ void boxCompute(const DiluView<T> &V, const int32_t *m, const Tile &t, Span sp, T *out,
                                            typename Bits<T>::U *inbox, Shared<T> &sh, unsigned &nSlow)
@@ -237,13 +253,16 @@ __device__ __forceinline__ void boxCompute(const DiluView<T> &V, const int32_t *
             for (int q = 0; q < 3; ++q)
                 if (!(FLAT && q == kSlotC)) y = y - p[q];
             if (!FULL) y = valid ? y : T(0);
-            plane[u][own] = y;
+            constexpr bool kMove = LONE && FLAT;
+            if (!kMove) plane[u][own] = y;
             // (other lanes' values are read back: not to be reordered, which
             // a lane's own addresses would allow)
             compilerFence();
             // the exchange comes first: its round trip is the step's chain,
             // and the stores below overlap it
-            if (u % kSub != kSub - 1) {
+            if (kMove) {
+                xb = laneBefore<T, kFwd>(y);
+            } else if (u % kSub != kSub - 1) {
                 xb = plane[u][nbB];
                 if (!FLAT) xc = plane[u][nbC];
             }
@@ -270,7 +289,7 @@ __device__ __forceinline__ void boxCompute(const DiluView<T> &V, const int32_t *
                 post(&sh.consumed, g + u + 1);
                 waitReady(g + u + 1 + kSub);
                 lookReady();
-                xb = plane[u][nbB];
+                if (!kMove) xb = plane[u][nbB];
                 if (!FLAT) xc = plane[u][nbC];
             }
             row[u % kLook] = getRow<T>(u + kLook < kG ? recG[u + kLook] : recN[u + kLook - kG], lane);
