@@ -483,6 +483,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     if (rounds.empty()) rounds.push_back(int2{0, 0});
     groups_.upload(groups, stream_);
     lvRounds_.upload(rounds, stream_);
+    lvProgress_.upload(std::vector<int32_t>(std::max(1, nGroups_), 0), stream_);
     nGenWaves_ = (int)order.size();
     nBoxWaves_ = (int)boxOrder.size();
     nBoxIn_ = boxIn;
@@ -699,6 +700,7 @@ DiluView<T> Batch::diluView(DevMatrix<T> &m, void *hF, void *hB)
     D.lvWaves = lvWaves_;
     D.lvDrain = lvDrain_;
     D.lvD = lvD_.p;
+    D.lvProgress = lvProgress_.p;
     D.boxInF = hF;
     D.boxInB = hB;
     D.boxInC = haloC64_.p;

@@ -394,7 +394,7 @@ private:
     std::vector<int32_t> hBoxMeta_, hBoxWaves_;   // host copies: box tile geometry, the box waves
     DevBuf<double> rdLocal_;                      // rD of the tile-local factor
     DevBuf<unsigned long long> rowMask_;   // per slice: lanes holding a cell
-    DevBuf<int32_t> fCodes_, bCodes_, fDeps_, bDeps_;
+    DevBuf<int32_t> fCodes_, bCodes_, fDeps_, bDeps_, lvProgress_;
     DevBuf<LevelGroup> groups_;
     DevBuf<int2> lvRounds_;
     DevBuf<double> lvD_;                          // d of the level groups' rows (factor)

@@ -211,6 +211,16 @@ __global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState 
 // bound here by one CU's load path (60 bytes a row in FP64, about 64 bytes a
 // clock) and the barrier.  Two regions of a system, or the systems of a batch,
 // run side by side on CUs of their own.
+//
+// One CU only has so many cache misses in flight: its rows came at 31 GB/s
+// (105 us a sweep of that mesh; 81 us with the helpers below), whatever the
+// depth.  So where few groups leave the chip idle, kHelpers more
+// workgroups per group, on the same XCD (workgroup b runs on XCD b mod kXcds;
+// elsewhere they only do not help), load the rows a little ahead of the sweep
+// and drop them: the sweep then hits the XCD's L2.
+constexpr int kXcds = 8, kHelpers = 8;
+constexpr int kWarmBytes = 3 << 19;   // of the 4 MB of L2
+
 template <int K>
 constexpr int kDeepOf = K <= 3 ? 3 : K <= 6 ? 2 : 1;
 
@@ -222,11 +232,17 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
     constexpr int G = packChunks(K + 1, N);
     constexpr int kDeep = kDeepOf<K>;
     __shared__ T ring[kLevelRing];
-    const LevelGroup g = V.groups[blockIdx.x];
+    // helper h of group g is workgroup kXcds + g + kXcds * h (launchGeneralK)
+    const bool helper = (int)blockIdx.x >= V.nGroups;
+    const int gi = helper ? (int)blockIdx.x % kXcds : (int)blockIdx.x;
+    if (helper && ((int)blockIdx.x < kXcds || gi >= V.nGroups)) return;
+    const LevelGroup g = V.groups[gi];
     if (MODE != kDiluFactor && st[g.sys].status != kRunning) return;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned long long tStart = V.trace ? wall_clock64() : 0ull;
-    const int2 *rounds = V.lvRounds + g.round0;
+    // (constant address space: scalar loads, which no wait for rows includes)
+    typedef const __attribute__((address_space(4))) int2 ConstInt2;
+    ConstInt2 *rounds = (ConstInt2 *)(V.lvRounds + __builtin_amdgcn_readfirstlane(g.round0));
     const int32_t *deps = MODE == kDiluBwd ? V.bDeps : V.fDeps;
     const R *recs = MODE == kDiluFactor ? (const R *)V.prodPack : (const R *)(MODE == kDiluBwd ? V.bPack : V.fPack);
     // what a later row reads back when it is out of the ring (the factor: d)
@@ -239,8 +255,12 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
         int s;       // the wave's slice, -1: none in this round
         int flags;
     };
-    auto load = [&](int i, Item &S) {
-        int2 r = rounds[MODE == kDiluBwd ? g.nRounds - 1 - min(i, g.nRounds - 1) : min(i, g.nRounds - 1)];
+    auto roundOf = [&](int i) {
+        i = min(i, g.nRounds - 1);
+        i = __builtin_amdgcn_readfirstlane(MODE == kDiluBwd ? g.nRounds - 1 - i : i);
+        return int2{rounds[i].x, rounds[i].y};
+    };
+    auto load = [&](int i, int2 r, Item &S) {
         const bool has = i < g.nRounds && wave < (r.y >> 2);
         const int s = r.x + (has ? wave : 0);   // (a slice to load from in any case: no load is conditional)
 #pragma unroll
@@ -251,31 +271,63 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
         S.s = has ? s : -1;
         S.flags = r.y & 3;
     };
-    Item buf[kDeep];
+    if (helper) {
+        // touch every kHelpers-th round's rows, at most kWarmBytes ahead of
+        // the sweep (the counter may still hold the last sweep's value, which
+        // only lets the first rounds run further ahead)
+        const int window = max(2 * kHelpers, kWarmBytes / (V.lvWaves * 64 * (int)(sizeof(R) * G + sizeof(int) * K + sizeof(T))));
+        for (int i = (int)blockIdx.x / kXcds - 1; i < g.nRounds; i += kHelpers) {
+            for (int spins = 0; spins < kPollLimit && i > __hip_atomic_load(&V.lvProgress[gi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + window; ++spins)
+                __builtin_amdgcn_s_sleep(8);
+            Item S;
+            load(i, roundOf(i), S);
 #pragma unroll
-    for (int u = 0; u < kDeep; ++u) load(u, buf[u]);
-    for (int i0 = 0; i0 < g.nRounds; i0 += kDeep) {
+            for (int q = 0; q < G; ++q) asm volatile("" ::"v"(elem(S.v[q], 0)));
 #pragma unroll
-        for (int u = 0; u < kDeep; ++u) {
+            for (int k = 0; k < K; ++k) asm volatile("" ::"v"(S.c[k]));
+            if (MODE != kDiluFactor) asm volatile("" ::"v"(S.a));
+        }
+        return;
+    }
+    // one slot more than rounds in flight: a round's rows are requested while
+    // the ring values of the current one are on their way (the round table's
+    // entry, a scalar load, one round earlier still)
+    constexpr int kSlots = kDeep + 1;
+    Item buf[kSlots];
+#pragma unroll
+    for (int u = 0; u < kDeep; ++u) load(u, roundOf(u), buf[u]);
+    int2 next = roundOf(kDeep);
+    for (int i0 = 0; i0 < g.nRounds; i0 += kSlots) {
+        if (V.lvHelped && threadIdx.x == 0)
+            __hip_atomic_store(&V.lvProgress[gi], i0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u) {
             const int i = i0 + u;
             Item &S = buf[u];
-            if (i < g.nRounds && S.s >= 0) {
+            const bool mine = i < g.nRounds && S.s >= 0;
+            T v[K];
+            if (mine) {
+#pragma unroll
+                for (int k = 0; k < K; ++k) v[k] = ring[S.c[k] & (kLevelRing - 1)];
+            }
+            load(i + kDeep, next, buf[(u + kDeep) % kSlots]);
+            next = roundOf(i + kDeep + 1);
+            if (mine) {
                 const T last = (T)elem(S.v[K / N], K % N);   // rD, or diag for the factor
-                T v[K];
                 bool far = false;
 #pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    far |= S.c[k] >= kLevelRing;
-                    v[k] = ring[S.c[k] & (kLevelRing - 1)];
-                }
+                for (int k = 0; k < K; ++k) far |= S.c[k] >= kLevelRing;
                 if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
                     // (stored more than kDeep rounds ago by a wave of this
                     // workgroup, which has waited since for loads issued
-                    // after that store: it has reached the CU's cache; the
-                    // factor reads the 1/d it stored, hence d's own copy)
+                    // after that store: it has reached the CU's cache)
 #pragma unroll
                     for (int k = 0; k < K; ++k)
                         if (S.c[k] >= kLevelRing) v[k] = MODE == kDiluFactor ? (T)V.lvD[(size_t)g.slice0 * 64 + S.c[k] - kLevelRing] : back[S.c[k] - kLevelRing];
+                    // (waited for here: after the branch the wait would cover
+                    // the rows in flight of every round)
+#pragma unroll
+                    for (int k = 0; k < K; ++k) asm volatile("" : "+v"(v[k]));
                 }
                 T y;
                 if (MODE == kDiluFwd) y = S.a * last;
@@ -302,9 +354,7 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
                     out[p] = y;
                 }
             }
-            const bool ends = i < g.nRounds && (S.flags & (MODE == kDiluBwd ? kRoundFirst : kRoundLast));
-            load(i + kDeep, S);
-            if (ends) {
+            if (i < g.nRounds && (S.flags & (MODE == kDiluBwd ? kRoundFirst : kRoundLast))) {
                 // the level's values are in the ring before any wave goes on.
                 // (Only LDS is waited for: a full fence would drain the rows
                 // in flight.  Values further back than the ring may be as
@@ -318,7 +368,7 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
         }
     }
     if (V.trace && threadIdx.x == 0) {
-        unsigned long long *tr = V.trace + 4 * ((size_t)V.nWaves + V.nBoxWaves + blockIdx.x);
+        unsigned long long *tr = V.trace + 4 * ((size_t)V.nWaves + V.nBoxWaves + gi);
         tr[0] = tStart;
         tr[1] = wall_clock64();
         tr[2] = 0;
@@ -532,7 +582,12 @@ template <typename T, int K, int MODE>
 static void launchGeneralK(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s)
 {
     if (V.nWaves > 0) k_dilu_wave<T, K, MODE><<<V.nWaves, 64, 0, s>>>(V, st, in, out);
-    if (V.nGroups > 0) k_dilu_levels<T, K, MODE><<<V.nGroups, 64 * V.lvWaves, 0, s>>>(V, st, in, out);
+    if (V.nGroups > 0) {
+        DiluView<T> L = V;
+        L.lvHelped = V.nGroups <= kXcds;
+        const int blocks = L.lvHelped ? kXcds * (1 + kHelpers) : V.nGroups;
+        k_dilu_levels<T, K, MODE><<<blocks, 64 * V.lvWaves, 0, s>>>(L, st, in, out);
+    }
 }
 
 template <typename T, int MODE>

@@ -64,6 +64,8 @@ struct DiluView {
     const int2 *lvRounds = nullptr;
     const int32_t *fDeps = nullptr, *bDeps = nullptr;
     int nGroups = 0, lvWaves = 1;
+    int *lvProgress = nullptr;           // per group: the round its sweep has reached
+    bool lvHelped = false;               // set by the launcher: helper workgroups read lvProgress
     bool lvDrain = false;                // a level is wider than a quarter of the ring
     double *lvD = nullptr;               // factor: d per row of the level groups
     typename Pack<T>::V *fPack = nullptr, *bPack = nullptr;
