@@ -268,7 +268,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     K_ = 3;
     for (auto &L : lay_) K_ = std::max(K_, roundK(L->K));
 
-    std::vector<int32_t> ellOff, ellCol, ifBase, ifRowFace, ifPairOff, ifPairCol;
+    std::vector<int32_t> ellOff, ellCol, sliceGeom, ifBase, ifRowFace, ifPairOff, ifPairCol;
     std::vector<unsigned long long> ifMask;
     std::vector<int32_t> cellOfPos, fCode, bCode, waveSlice, waveSteps, waveSys;
     std::vector<const std::vector<int32_t> *> waveLevels;
@@ -294,6 +294,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
             ifMask.push_back(L.ifMask[s]);
         }
         appendShift(ellCol, L.ellCol, pos0);
+        sliceGeom.insert(sliceGeom.end(), L.sliceGeom.begin(), L.sliceGeom.end());
         appendShift(ifPairCol, L.ifPairCol, pos0);
         for (size_t i = 0; i + 1 < L.ifRowFace.size(); ++i) ifRowFace.push_back(L.ifRowFace[i] + ifFaceBase);
         for (size_t i = 0; i + 1 < L.ifPairOff.size(); ++i) ifPairOff.push_back(L.ifPairOff[i] + ifPairBase);
@@ -523,6 +524,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     hipStream_t st = stream_;
     ellOff_.upload(ellOff, st);
     ellCol_.upload(ellCol, st);
+    sliceGeom_.upload(sliceGeom, st);
     ifMask_.upload(ifMask, st);
     ifBase_.upload(ifBase, st);
     ifRowFace_.upload(ifRowFace, st);
@@ -652,6 +654,7 @@ MatView<T> Batch::view(const DevMatrix<T> &m) const
     MatView<T> A;
     A.ellOff = ellOff_.p;
     A.ellCol = ellCol_.p;
+    A.sliceGeom = sliceGeom_.p;
     A.ellVal = m.ellVal.p;
     A.diag = m.diag.p;
     A.ifMask = ifMask_.p;

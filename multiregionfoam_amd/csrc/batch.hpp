@@ -373,7 +373,7 @@ private:
     }
 
     // structure (shared by both precisions)
-    DevBuf<int32_t> ellOff_, ellCol_, ifBase_, ifRowFace_, ifPairOff_, ifPairCol_;
+    DevBuf<int32_t> ellOff_, ellCol_, sliceGeom_, ifBase_, ifRowFace_, ifPairOff_, ifPairCol_;
     DevBuf<unsigned long long> ifMask_;
     DevBuf<int32_t> cellOfPos_;
     DevBuf<BlockEntry> blocks_;

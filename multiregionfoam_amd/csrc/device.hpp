@@ -40,6 +40,7 @@ template <typename T>
 struct MatView {
     const int32_t *ellOff;
     const int32_t *ellCol;
+    const int32_t *sliceGeom;   // kSliceGeom ints per slice (layout.hpp)
     const T *ellVal;
     const T *diag;
     const unsigned long long *ifMask;

@@ -394,6 +394,27 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
         }
     }
 
+    // ---- geometry of the 3-D box slices (the columns of their SpMV entries) ----
+    L.sliceGeom.assign((size_t)L.nSlices * kSliceGeom, 0);
+    for (int s = 0; s < L.nSlices; ++s) L.sliceGeom[(size_t)s * kSliceGeom + kSgAxis] = -1;
+    for (int wi = 0; wi < L.nWaves; ++wi) {
+        if (!L.waveBox[wi]) continue;
+        const RegionSchedule &rs = L.schedules[waves[ord[wi]].region];
+        if (rs.n[0] < 2 || rs.n[1] < 2 || rs.n[2] < 2) continue;
+        const int32_t *m = &L.boxMeta[(size_t)wi * kBoxMeta];
+        const int TB = m[kBmTB], TC = kSlice / TB;
+        // lane l's row of step t is cell ia = t - bl - cl of its line, in the
+        // tile and in its neighbours alike
+        auto across = [&](int to, int dStep, int dLane) {
+            return m[to] < 0 ? 0 : (L.waveSlice[m[to]] - L.waveSlice[wi] + dStep) * kSlice + dLane;
+        };
+        const int g[kSliceGeom] = {m[kBmAxis], __builtin_ctz(TB), across(kBmPrevB, TB - 1, TB - 1),
+                                   across(kBmNextB, 1 - TB, 1 - TB), across(kBmPrevC, TC - 1, TB * (TC - 1)),
+                                   across(kBmNextC, 1 - TC, -TB * (TC - 1)), 0, 0};
+        for (int t = 0; t < L.waveSteps[wi]; ++t)
+            std::copy(g, g + kSliceGeom, &L.sliceGeom[(size_t)(L.waveSlice[wi] + t) * kSliceGeom]);
+    }
+
     // ---- per-slice ELL (SpMV) ----
     L.ellOff.assign(L.nSlices + 1, 0);
     L.ifMask.assign(L.nSlices, 0);
@@ -407,6 +428,7 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
             if (c < 0) continue;
             wE = std::max(wE, (D.lo_off[c + 1] - D.lo_off[c]) + (D.up_off[c + 1] - D.up_off[c]));
         }
+        if (L.sliceGeom[(size_t)s * kSliceGeom + kSgAxis] >= 0) wE = 6;
         L.ellOff[s + 1] = L.ellOff[s] + wE;
     }
     L.ellCol.assign((size_t)L.ellOff[L.nSlices] * kSlice, 0);
@@ -450,13 +472,21 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
             auto loSrc = [&](int f) { return 2 * (L.faceOffset[r] + f) + (R.symmetric ? 1 : 0); };
             auto upSrc = [&](int f) { return 2 * (L.faceOffset[r] + f) + 1; };
             int k = 0;
+            // the entry of a 3-D box row is that of the neighbour's axis
+            const bool byAxis = L.sliceGeom[(size_t)s * kSliceGeom + kSgAxis] >= 0;
+            auto axisOf = [&](int d) {
+                const RegionSchedule &rs = L.schedules[r];
+                return d == 1 ? 0 : d == rs.n[0] ? 1 : 2;
+            };
             for (int q = D.lo_off[c]; q < D.lo_off[c + 1]; ++q, ++k) {
+                if (byAxis) k = 2 - axisOf(c - D.lo_nb[q]);
                 size_t e = (size_t)(L.ellOff[s] + k) * kSlice + l;
                 L.ellCol[e] = L.posOfCell[D.lo_nb[q]];
                 L.ellVal[e] = lo[D.lo_face[q]];
                 L.ellSrc[e] = loSrc(D.lo_face[q]);
             }
             for (int q = D.up_off[c]; q < D.up_off[c + 1]; ++q, ++k) {
+                if (byAxis) k = 3 + axisOf(D.up_nb[q] - c);
                 size_t e = (size_t)(L.ellOff[s] + k) * kSlice + l;
                 L.ellCol[e] = L.posOfCell[D.up_nb[q]];
                 L.ellVal[e] = R.upper[D.up_face[q]];

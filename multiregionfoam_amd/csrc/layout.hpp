@@ -72,6 +72,11 @@ enum {
     kBoxMeta = 16
 };
 
+// Per-slice geometry: the sequential axis (-1: not a 3-D box tile, the columns
+// are listed), log2 of TB, and for the rows on the tile's edges the distance to
+// the neighbour's position across it (0: none).
+enum { kSgAxis = 0, kSgLogTB, kSgPrevB, kSgNextB, kSgPrevC, kSgNextC, kSliceGeom = 8 };
+
 struct RegionSchedule {
     std::string kind;                // "box", "chain" or "levels"
     int n[3] = {0, 0, 0};            // box dimensions
@@ -92,6 +97,11 @@ struct SystemLayout {
     std::vector<int32_t> ellOff;             // nSlices + 1, in 64-entry columns
     std::vector<int32_t> ellCol;
     std::vector<double> ellVal;
+    // per slice, kSliceGeom ints: where the neighbours of a 3-D box tile's
+    // rows are.  Such a slice has six entries per row in the order of the
+    // axes (z, y, x lower, then x, y, z upper; zero where there is none), so
+    // their columns follow from the tile
+    std::vector<int32_t> sliceGeom;
     std::vector<double> diag, source, sumA, psi0;
     // GGI interface rows
     std::vector<uint64_t> ifMask;            // per slice
