@@ -500,9 +500,24 @@ __device__ __forceinline__ void boxFactor(const DiluView<double> &V, const int32
                 // a sentinel (a NaN) makes the value NaN; a second pass
                 // follows the wait for the late values
                 if (LONE || pass || __builtin_expect(__builtin_amdgcn_ballot_w64(yz != yz) == 0, 1)) break;
+                // poll rounds: each reloads this step's values and those
+                // already requested for the next steps, all in flight
+                // together; the later ones come with the last round instead
+                // of a round trip each (145 -> 240 us a factor of the 1.4M
+                // cell duct without)
                 for (int spins = 0;; ++spins) {
-                    S.hb = S.hb == kSent ? haloLoad(myIn + (size_t)stepOf(i) * TBC, cl) : S.hb;
-                    S.hc = S.hc == kSent ? haloLoad(myIn + (size_t)stepOf(i) * TBC, TC + bl) : S.hc;
+                    U nb[kFacInAhead], nc[kFacInAhead];
+#pragma unroll
+                    for (int k = 0; k < kFacInAhead; ++k) {
+                        nb[k] = haloLoad(myIn + (size_t)stepOf(i + k) * TBC, cl);
+                        nc[k] = haloLoad(myIn + (size_t)stepOf(i + k) * TBC, TC + bl);
+                    }
+#pragma unroll
+                    for (int k = 0; k < kFacInAhead; ++k) {
+                        Step &F = buf[(u + k) % kFacAhead];
+                        F.hb = F.hb == kSent ? nb[k] : F.hb;
+                        F.hc = F.hc == kSent ? nc[k] : F.hc;
+                    }
                     const bool late = valid && ((useB && S.hb == kSent) || (useC && S.hc == kSent));
                     if (__builtin_amdgcn_ballot_w64(late) == 0) break;
                     // an expired wait ends every later one at once, so a
