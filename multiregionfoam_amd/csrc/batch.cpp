@@ -67,7 +67,7 @@ template struct DevBuf<int32_t>;
 template struct DevBuf<unsigned long long>;
 template struct DevBuf<int8_t>;
 template struct DevBuf<LevelGroup>;
-template struct DevBuf<int2>;
+template struct DevBuf<LevelRound>;
 template struct DevBuf<FvRegionParams>;
 template struct DevBuf<DnaSide>;
 template struct DevBuf<DnaCell>;
@@ -272,6 +272,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     std::vector<unsigned long long> ifMask;
     std::vector<int32_t> cellOfPos, fCode, bCode, waveSlice, waveSteps, waveSys;
     std::vector<const std::vector<int32_t> *> waveLevels;
+    std::vector<uint8_t> waveFar;
     std::vector<double> diag, source, sumA, psi0, fProd;
     std::vector<std::array<int, 3>> waveKey;   // (key, system, global wave index)
     std::vector<uint8_t> waveBox;
@@ -349,6 +350,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
             waveSys.push_back(q);
             waveBox.push_back(L.waveBox[w]);
             waveLevels.push_back(&L.waveLevels[w]);
+            waveFar.push_back(L.waveFar[w]);
             // box tile geometry with batch-wide wave, slice and inbox indices
             const int32_t *lm = &L.boxMeta[(size_t)w * kBoxMeta];
             std::array<int32_t, kBoxMeta> gm;
@@ -464,24 +466,17 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     for (int w : grouped)
         for (int n : *waveLevels[w]) widest = std::max(widest, n);
     lvWaves_ = std::min(16, widest);
-    lvDrain_ = widest * kSlice > kLevelRing / 4;
     std::vector<LevelGroup> groups;
-    std::vector<int2> rounds;
+    std::vector<LevelRound> rounds;
     for (int w : grouped) {
         LevelGroup g{waveSlice[w], (int)rounds.size(), 0, waveSys[w]};
-        int s = waveSlice[w];
-        for (int n : *waveLevels[w])
-            for (int k = 0; k < n; k += lvWaves_) {
-                const int cnt = std::min(lvWaves_, n - k);
-                rounds.push_back(int2{s, cnt << 2 | (k + cnt == n ? kRoundLast : 0) | (k == 0 ? kRoundFirst : 0)});
-                s += cnt;
-            }
+        levelRounds(*waveLevels[w], waveSlice[w], lvWaves_, waveFar[w] != 0, rounds);
         g.nRounds = (int)rounds.size() - g.round0;
         groups.push_back(g);
     }
     nGroups_ = (int)groups.size();
     if (groups.empty()) groups.push_back(LevelGroup{});
-    if (rounds.empty()) rounds.push_back(int2{0, 0});
+    if (rounds.empty()) rounds.push_back(LevelRound{0, 0});
     groups_.upload(groups, stream_);
     lvRounds_.upload(rounds, stream_);
     lvProgress_.upload(std::vector<int32_t>(std::max(1, nGroups_), 0), stream_);
@@ -701,7 +696,6 @@ DiluView<T> Batch::diluView(DevMatrix<T> &m, void *hF, void *hB)
     D.bDeps = bDeps_.p;
     D.nGroups = nGroups_;
     D.lvWaves = lvWaves_;
-    D.lvDrain = lvDrain_;
     D.lvD = lvD_.p;
     D.lvProgress = lvProgress_.p;
     D.boxInF = hF;

@@ -396,10 +396,9 @@ private:
     DevBuf<unsigned long long> rowMask_;   // per slice: lanes holding a cell
     DevBuf<int32_t> fCodes_, bCodes_, fDeps_, bDeps_, lvProgress_;
     DevBuf<LevelGroup> groups_;
-    DevBuf<int2> lvRounds_;
+    DevBuf<LevelRound> lvRounds_;
     DevBuf<double> lvD_;                          // d of the level groups' rows (factor)
     int nGroups_ = 0, lvWaves_ = 1;
-    bool lvDrain_ = false;
     DevBuf<double2> prodPack_;
     DevBuf<unsigned long long> haloF64_, haloB64_, haloC64_;
     DevBuf<unsigned int> haloF32_, haloB32_;

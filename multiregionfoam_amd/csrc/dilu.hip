@@ -241,8 +241,8 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned long long tStart = V.trace ? wall_clock64() : 0ull;
     // (constant address space: scalar loads, which no wait for rows includes)
-    typedef const __attribute__((address_space(4))) int2 ConstInt2;
-    ConstInt2 *rounds = (ConstInt2 *)(V.lvRounds + __builtin_amdgcn_readfirstlane(g.round0));
+    typedef const __attribute__((address_space(4))) LevelRound ConstRound;
+    ConstRound *rounds = (ConstRound *)(V.lvRounds + __builtin_amdgcn_readfirstlane(g.round0));
     const int32_t *deps = MODE == kDiluBwd ? V.bDeps : V.fDeps;
     const R *recs = MODE == kDiluFactor ? (const R *)V.prodPack : (const R *)(MODE == kDiluBwd ? V.bPack : V.fPack);
     // what a later row reads back when it is out of the ring (the factor: d)
@@ -258,18 +258,18 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
     auto roundOf = [&](int i) {
         i = min(i, g.nRounds - 1);
         i = __builtin_amdgcn_readfirstlane(MODE == kDiluBwd ? g.nRounds - 1 - i : i);
-        return int2{rounds[i].x, rounds[i].y};
+        return LevelRound{rounds[i].slice, rounds[i].word};
     };
-    auto load = [&](int i, int2 r, Item &S) {
-        const bool has = i < g.nRounds && wave < (r.y >> 2);
-        const int s = r.x + (has ? wave : 0);   // (a slice to load from in any case: no load is conditional)
+    auto load = [&](int i, LevelRound r, Item &S) {
+        const bool has = i < g.nRounds && wave < (r.word >> kRoundBits);
+        const int s = r.slice + (has ? wave : 0);   // (a slice to load from in any case: no load is conditional)
 #pragma unroll
         for (int q = 0; q < G; ++q) S.v[q] = recs[((size_t)s * G + q) * 64 + lane];
 #pragma unroll
         for (int k = 0; k < K; ++k) S.c[k] = deps[((size_t)s * K + k) * 64 + lane];
         if (MODE != kDiluFactor) S.a = in[(size_t)s * 64 + lane];
         S.s = has ? s : -1;
-        S.flags = r.y & 3;
+        S.flags = r.word & ((1 << kRoundBits) - 1);
     };
     if (helper) {
         // touch every kHelpers-th round's rows, at most kWarmBytes ahead of
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
     Item buf[kSlots];
 #pragma unroll
     for (int u = 0; u < kDeep; ++u) load(u, roundOf(u), buf[u]);
-    int2 next = roundOf(kDeep);
+    LevelRound next = roundOf(kDeep);
     for (int i0 = 0; i0 < g.nRounds; i0 += kSlots) {
         if (V.lvHelped && threadIdx.x == 0)
             __hip_atomic_store(&V.lvProgress[gi], i0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -318,14 +318,15 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
 #pragma unroll
                 for (int k = 0; k < K; ++k) far |= S.c[k] >= kLevelRing;
                 if (__builtin_expect(__builtin_amdgcn_ballot_w64(far) != 0, 0)) {
-                    // (stored more than kDeep rounds ago by a wave of this
-                    // workgroup, which has waited since for loads issued
-                    // after that store: it has reached the CU's cache)
+                    // (in memory: a barrier that waits for stores lies
+                    // between the row's level and this one, levelRounds.
+                    // Such a load waits for the rows in flight as well, which
+                    // are counted before it.)
 #pragma unroll
                     for (int k = 0; k < K; ++k)
                         if (S.c[k] >= kLevelRing) v[k] = MODE == kDiluFactor ? (T)V.lvD[(size_t)g.slice0 * 64 + S.c[k] - kLevelRing] : back[S.c[k] - kLevelRing];
-                    // (waited for here: after the branch the wait would cover
-                    // the rows in flight of every round)
+                    // (waited for here: after the branch every round would
+                    // wait for its rows in flight, also one without such a row)
 #pragma unroll
                     for (int k = 0; k < K; ++k) asm volatile("" : "+v"(v[k]));
                 }
@@ -356,11 +357,9 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
             }
             if (i < g.nRounds && (S.flags & (MODE == kDiluBwd ? kRoundFirst : kRoundLast))) {
                 // the level's values are in the ring before any wave goes on.
-                // (Only LDS is waited for: a full fence would drain the rows
-                // in flight.  Values further back than the ring may be as
-                // recent as the last level only where levels are wider than
-                // a quarter of it: there the stores are waited for too.)
-                if (V.lvDrain) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                // (Where no row is about to leave the ring only LDS is waited
+                // for: waiting for the stores drains the rows in flight.)
+                if (S.flags & (MODE == kDiluBwd ? kRoundStoredB : kRoundStoredF)) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
                 else asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");

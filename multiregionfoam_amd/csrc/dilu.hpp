@@ -45,9 +45,8 @@ struct Pack<float> {
 constexpr int packChunks(int n, int per) { return (n + per - 1) / per; }
 constexpr int kCodeNone = 0xFF;
 
-// One workgroup's sweep of a level group: rounds of up to lvWaves slices, the
-// first slice and (count << 2 | flags) of each in `lvRounds`
-enum { kRoundLast = 1, kRoundFirst = 2 };   // the round ends / starts a level
+// One workgroup's sweep of a level group: rounds of up to lvWaves slices
+// (layout.hpp, LevelRound)
 struct LevelGroup {
     int slice0, round0, nRounds, sys;
 };
@@ -61,12 +60,11 @@ struct DiluView {
     const int32_t *fCodes = nullptr, *bCodes = nullptr;
     // level groups
     const LevelGroup *groups = nullptr;
-    const int2 *lvRounds = nullptr;
+    const LevelRound *lvRounds = nullptr;
     const int32_t *fDeps = nullptr, *bDeps = nullptr;
     int nGroups = 0, lvWaves = 1;
     int *lvProgress = nullptr;           // per group: the round its sweep has reached
     bool lvHelped = false;               // set by the launcher: helper workgroups read lvProgress
-    bool lvDrain = false;                // a level is wider than a quarter of the ring
     double *lvD = nullptr;               // factor: d per row of the level groups
     typename Pack<T>::V *fPack = nullptr, *bPack = nullptr;
     const double2 *prodPack = nullptr;   // factor records (FP64)

@@ -185,6 +185,39 @@ bool detectBox(const LduRegion &R, int n[3])
     return true;
 }
 
+// A row beyond the ring is read back from memory, so a barrier that waits for
+// stores has to lie between its level and the reader's.  One such barrier at
+// each level end where the rows since the last one and the next level's would
+// exceed the ring is enough: if a forward row of level A had none before its
+// reader's level L, all rows from A's first to L's last would fit the ring, and
+// the row would be read from there (backward alike).
+void levelRounds(const std::vector<int32_t> &levels, int slice0, int waves, bool far, std::vector<LevelRound> &out)
+{
+    const int nL = (int)levels.size();
+    std::vector<int> stored(nL, 0);
+    constexpr int kMost = kLevelRing / kSlice;
+    long long sum = 0;
+    for (int lv = 0; far && lv + 1 < nL; ++lv) {
+        sum += levels[lv];
+        if (sum + levels[lv + 1] > kMost) stored[lv] |= kRoundStoredF, sum = 0;
+    }
+    sum = 0;
+    for (int lv = nL - 1; far && lv > 0; --lv) {
+        sum += levels[lv];
+        if (sum + levels[lv - 1] > kMost) stored[lv] |= kRoundStoredB, sum = 0;
+    }
+    int s = slice0;
+    for (int lv = 0; lv < nL; ++lv)
+        for (int k = 0; k < levels[lv]; k += waves) {
+            const int cnt = std::min(waves, levels[lv] - k);
+            int flags = 0;
+            if (k + cnt == levels[lv]) flags |= kRoundLast | (stored[lv] & kRoundStoredF);
+            if (k == 0) flags |= kRoundFirst | (stored[lv] & kRoundStoredB);
+            out.push_back({s, cnt << kRoundBits | flags});
+            s += cnt;
+        }
+}
+
 SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
 {
     sys.check();
@@ -254,6 +287,7 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
     L.waveSteps.resize(L.nWaves);
     L.waveKey.resize(L.nWaves);
     L.waveLevels.resize(L.nWaves);
+    L.waveFar.assign(L.nWaves, 0);
     int slice = 0;
     for (int wi = 0; wi < L.nWaves; ++wi) {
         const WaveBuild &w = waves[ord[wi]];
@@ -535,7 +569,9 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
                         if (lvEnd[pd / kSlice] > lvBegin[s]) throw std::runtime_error("DILU schedule violates a forward dependency");
                         // in the ring until the rows kLevelRing further on are written
                         const int at = td * kSlice + ld;
-                        L.fCode[e] = lvEnd[s] * kSlice - at <= kLevelRing ? at & (kLevelRing - 1) : kLevelRing + at;
+                        const bool far = lvEnd[s] * kSlice - at > kLevelRing;
+                        L.fCode[e] = far ? kLevelRing + at : at & (kLevelRing - 1);
+                        if (far) L.waveFar[w] = 1;
                     } else {
                         if (t - td < 1 || t - td > kRing - 1) throw std::runtime_error("DILU schedule violates a forward dependency");
                         L.fCode[e] = (td % kRing) * kSlice + ld;
@@ -555,7 +591,9 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
                     if (lvEnd[s] >= 0) {
                         if (lvBegin[pd / kSlice] < lvEnd[s]) throw std::runtime_error("DILU schedule violates a backward dependency");
                         const int at = td * kSlice + ld;
-                        L.bCode[e] = at - lvBegin[s] * kSlice < kLevelRing ? at & (kLevelRing - 1) : kLevelRing + at;
+                        const bool far = at - lvBegin[s] * kSlice >= kLevelRing;
+                        L.bCode[e] = far ? kLevelRing + at : at & (kLevelRing - 1);
+                        if (far) L.waveFar[w] = 1;
                     } else {
                         if (td - t < 1 || td - t > kRing - 1) throw std::runtime_error("DILU schedule violates a backward dependency");
                         L.bCode[e] = ((T - 1 - td) % kRing) * kSlice + ld;

@@ -54,6 +54,20 @@ constexpr int kRing = 3;            // LDS ring depth (steps) of a DILU wave (sl
 constexpr int32_t kNoDep = -1;
 constexpr int kLevelRing = 16384;   // rows of a level group's LDS ring (128 KB in FP64); a power of two
 
+// A round of a level group's workgroup: the slices of one level that it takes
+// side by side, one per wave.
+struct LevelRound {
+    int32_t slice;   // the first
+    int32_t word;    // their number << kRoundBits | flags
+};
+enum {
+    kRoundLast = 1,      // ends its level: a barrier follows (forward)
+    kRoundFirst = 2,     // starts its level: a barrier follows (backward)
+    kRoundStoredF = 4,   // at that barrier the rows stored so far have to be
+    kRoundStoredB = 8,   // in memory (forward / backward)
+    kRoundBits = 4
+};
+
 // Per-wave metadata of a structured-box tile wave (kBoxMeta ints each).
 enum {
     kBmTB = 0,      // lanes along the tile's first tangential axis (TC = 64/TB)
@@ -116,6 +130,7 @@ struct SystemLayout {
     std::vector<double> fVal, fProd, bVal;
     // per wave: the slices of each level of a level group (empty for others)
     std::vector<std::vector<int32_t>> waveLevels;
+    std::vector<uint8_t> waveFar;            // per wave: 1 if a dependency lies beyond the LDS ring
     // structured-box tile waves: their rows keep the DILU values in fixed
     // slots (slot = 2 - axis of the neighbour: z, y, x, which is both the
     // face order of the lower neighbours and the reverse face order of the
@@ -137,6 +152,11 @@ struct SystemLayout {
 // Build the layout.  `preferLevels` forces the level schedule for every
 // region (used to test the general path on structured meshes).
 SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels = false);
+
+// Append the rounds of a level group of `levels` (slices per level) from
+// slice0 on, for workgroups of `waves` waves; `far`: with dependencies beyond
+// the LDS ring, whose rows the marked barriers put into memory in time.
+void levelRounds(const std::vector<int32_t> &levels, int slice0, int waves, bool far, std::vector<LevelRound> &out);
 
 // Detect a lexicographically numbered structured hex box from LDU
 // addressing; returns false if the region is not one.

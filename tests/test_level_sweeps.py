@@ -52,6 +52,29 @@ def graph(N, most, seed=6):
                 diag=diag, source=rng.standard_normal(N), psi=rng.standard_normal(N))
 
 
+def ladder(widths, seed=8):
+    """Levels of the given widths: each cell has a lower neighbour in the
+    level before its own (at most six to one), and most of those from the 20th
+    level on one among the first cells as well."""
+    rng = np.random.default_rng(seed)
+    start = np.concatenate([[0], np.cumsum(widths)])
+    faces, up = set(), np.zeros(start[-1], dtype=int)
+    for lv in range(1, len(widths)):
+        for i in range(widths[lv]):
+            c = int(start[lv]) + i
+            before = int(start[lv - 1]) + (i % widths[lv - 1])
+            far = int(rng.integers(0, start[min(20, lv)]))
+            for l in (before, far) if lv >= 20 and up[far] < 5 else (before,):
+                faces.add((l, c))
+                up[l] += 1
+    f = np.array(sorted(faces), dtype=np.int32)
+    u, lo = -rng.uniform(0.1, 1.0, len(f)), -rng.uniform(0.1, 1.0, len(f))
+    N = int(start[-1])
+    diag = 0.5 - np.bincount(f[:, 0], u, N) - np.bincount(f[:, 1], lo, N)
+    return dict(nCells=N, nFaces=len(f), symmetric=False, lAddr=f[:, 0].copy(), uAddr=f[:, 1].copy(), lower=lo, upper=u,
+                diag=diag, source=rng.standard_normal(N), psi=rng.standard_normal(N))
+
+
 def strip():
     """Three blocks side by side, numbered one after the other: a chain."""
     n = (60, 20, 1)
@@ -65,6 +88,9 @@ CASES = {
     "narrow_levels": lambda: [front((23, 11, 9), 0.9)],
     "levels_over_a_workgroup": lambda: [front((60, 45, 40), 0.5), front((40, 33, 9), 2.5)],
     "beyond_the_ring": lambda: [shuffled((40, 40, 30))],
+    # a wide level, then levels that most waves of the workgroup have no part
+    # in, with rows read back long after they have left the ring
+    "far_rows_of_narrow_levels": lambda: [ladder([1000] + [300] * 110), ladder([2000, 700] + [64] * 300 + [300] + [900] * 5)],
     "six_neighbours": lambda: [shuffled((13, 11, 7))],
     "twelve_neighbours": lambda: [graph(1500, 12), front((17, 9, 8), 0.5)],
     "with_chain_and_box": lambda: [strip(), box((30, 17, 5), 8), front((12, 12, 12), 0.9)],
