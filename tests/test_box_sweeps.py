@@ -30,7 +30,12 @@ def box(n, seed, symmetric=False):
                 psi=rng.standard_normal(N))
 
 
-@pytest.mark.parametrize("n", SHAPES, ids=lambda n: "x".join(map(str, n)))
+# boxes of several flat or nearly flat tiles, whose inboxes have sides that no
+# neighbour delivers to
+FLAT = [(300, 66, 1), (70, 300, 1), (1, 90, 150), (200, 130, 2), (64, 200, 3), (3, 70, 400)]
+
+
+@pytest.mark.parametrize("n", SHAPES + FLAT, ids=lambda n: "x".join(map(str, n)))
 def test_sweeps_match_oracle(gpu, n):
     # two boxes in one system, so that tiles of both are swept by one launch
     regions = [box(n, 1), box((n[0], n[2], n[1]), 2, symmetric=True)]
