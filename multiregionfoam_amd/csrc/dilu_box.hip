@@ -441,9 +441,11 @@ __device__ __forceinline__ void boxFeed(const DiluView<T> &V, const int32_t *m, 
     int nb = firstB + (lane >> (6 - LG)), nc = firstC + (lane >> LG);
     // inbox rows by step: step i is row T = i (forward) / nL - 1 - i.  (A
     // row outside the inbox is not loaded, the hardware returns zero, and it
-    // is never taken.)
-    const auto rB = rawBuffer(inbox + t.inbox, (size_t)nL * kRow);
-    const auto rC = rawBuffer(inbox + t.inbox + (size_t)nL * E, (size_t)nL * kRow);
+    // is never taken.  Nor is any row of a side without a neighbour, which a
+    // flat tile would ask for eight full rows of in each batch: a fed tile of
+    // 1000x66 cells went at 145 ns a step.)
+    const auto rB = rawBuffer(inbox + t.inbox, prevB ? (size_t)nL * kRow : 0);
+    const auto rC = rawBuffer(inbox + t.inbox + (size_t)nL * E, prevC ? (size_t)nL * kRow : 0);
     auto offsetOf = [&](int i, int v) { return (unsigned)((kFwd ? i : nL - 1 - i) * kRow + v * (int)sizeof(U)); };
     // where they go: the plane of the step before
     U *toB = (U *)&sh.plane[0][t.cell<kFwd>(kFwd ? -1 : TB, cv)], *toC = (U *)&sh.plane[0][t.cell<kFwd>(bv, kFwd ? -1 : TC)];
