@@ -453,6 +453,10 @@ int mrfg_tuning(mrfg_ctx *ctx, int *tuned, int *block_threads, int *ell_chunk, d
    2, 4, 8 or 16) for the following solves of the committed batch, as if the
    autotuner had chosen it (testing and profiling facility). */
 int mrfg_set_tuning(mrfg_ctx *ctx, int block_threads, int ell_chunk);
+/* Polls (1 to 2^20, the default: about a second) after which one wait of a
+   DILU sweep for a neighbouring tile fails the call instead of waiting on,
+   for the following calls on the committed batch (testing facility). */
+int mrfg_set_wait_limit(mrfg_ctx *ctx, int polls);
 /* info[0..5] = cells, internal faces, GGI pairs, rows incl. padding,
    64-row slices, DILU waves. */
 int mrfg_layout_info(mrfg_ctx *ctx, int sys, long long *info);

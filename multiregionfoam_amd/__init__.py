@@ -129,6 +129,7 @@ def lib():
         "mrfg_layout_info": ([vp, C.c_int, C.POINTER(C.c_longlong)], C.c_int),
         "mrfg_tuning": ([vp, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int), F64P, F64P], C.c_int),
         "mrfg_set_tuning": ([vp, C.c_int, C.c_int], C.c_int),
+        "mrfg_set_wait_limit": ([vp, C.c_int], C.c_int),
         "mrfg_trace_dilu": ([vp, C.POINTER(C.c_longlong), C.c_int, C.POINTER(C.c_int)], C.c_int),
         "mrfg_bytes": ([vp, C.c_int, C.c_int, F64P, F64P, F64P], C.c_int),
         "mrfg_copy_probe": ([vp, C.c_longlong, C.c_int, F64P], C.c_int),
@@ -167,7 +168,7 @@ EXPORTED = (
     "mrfg_case_region_source_base "
     "mrfg_case_interface_sizes mrfg_case_interface mrfg_case_interface_wall mrfg_set_interface_wall "
     "mrfg_interface_patch_values mrfg_add_case mrfg_spmv mrfg_dilu_factor "
-    "mrfg_precondition mrfg_precondition_fp32 mrfg_precondition_inner mrfg_dilu_tiles mrfg_time_kernel mrfg_trace_dilu mrfg_layout_info mrfg_tuning mrfg_set_tuning mrfg_bytes mrfg_copy_probe mrfg_interface_flux mrfg_interface_flux_noalloc "
+    "mrfg_precondition mrfg_precondition_fp32 mrfg_precondition_inner mrfg_dilu_tiles mrfg_time_kernel mrfg_trace_dilu mrfg_layout_info mrfg_tuning mrfg_set_tuning mrfg_set_wait_limit mrfg_bytes mrfg_copy_probe mrfg_interface_flux mrfg_interface_flux_noalloc "
     "mrfg_set_field mrfg_assemble mrfg_get_region_matrix mrfg_get_interface_coeff mrfg_assembly_bytes "
     "mrfg_server_create mrfg_server_destroy mrfg_server_submit mrfg_server_wait_all mrfg_server_result "
     "mrfg_server_get_psi mrfg_server_times mrfg_server_last_error").split()
@@ -723,6 +724,10 @@ class CoupledFvMatrix:
     def set_tuning(self, block_threads, ell_chunk):
         """Force a launch configuration for the following solves."""
         self._check(lib().mrfg_set_tuning(self._h, int(block_threads), int(ell_chunk)))
+
+    def set_wait_limit(self, polls):
+        """Polls after which one wait of a DILU sweep fails the call."""
+        self._check(lib().mrfg_set_wait_limit(self._h, int(polls)))
 
     def bytes_model(self, sys=0, value_size=8):
         a, b, c = C.c_double(), C.c_double(), C.c_double()

@@ -702,6 +702,7 @@ DiluView<T> Batch::diluView(DevMatrix<T> &m, void *hF, void *hB)
     D.boxInB = hB;
     D.boxInC = haloC64_.p;
     D.err = err_.p;
+    D.waitLimit = waitLimit_;
     D.side = side_;
     D.fork = fork_;
     D.join = join_;

@@ -239,6 +239,11 @@ public:
         setTuning(slices, ellChunk);
         tune_.tuned = true;
     }
+    void setWaitLimit(int polls)
+    {
+        waitLimit_ = polls;
+        dropGraphs();   // the captured launches hold the previous limit
+    }
     // device field and right-hand side (batch positions) and the position of
     // global cell `cell` of system `sys`
     const double *fieldDevice() const { return x64_.p; }
@@ -355,6 +360,7 @@ private:
     std::vector<int> sliceBegin_;
     int nSlices_ = 0, nPos_ = 0, nBlk_ = 0, nWaves_ = 0, K_ = 3;
     int nGenWaves_ = 0, nBoxWaves_ = 0, nBoxIn_ = 0;
+    int waitLimit_ = kWaitLimit;
     bool boxLone_ = false;   // every box tile alone in its region
     bool factorised_ = false, haveFloat_ = false;
     bool tileLocal32_ = false;   // the FP32 records are those of the tile-local DILU

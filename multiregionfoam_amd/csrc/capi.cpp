@@ -760,6 +760,15 @@ int mrfg_set_tuning(mrfg_ctx *ctx, int block_threads, int ell_chunk)
     });
 }
 
+int mrfg_set_wait_limit(mrfg_ctx *ctx, int polls)
+{
+    if (!ctx) return MRFG_ERR_ARG;
+    return guard(ctx, [&] {
+        if (polls < 1 || polls > mrfg::kWaitLimit) throw ArgError("polls must be between 1 and " + std::to_string(mrfg::kWaitLimit));
+        committedBatch(ctx).setWaitLimit(polls);
+    });
+}
+
 int mrfg_interface_flux(mrfg_ctx *ctx, int sys, int iface, double *q_a, double *q_b)
 {
     if (!ctx || !q_a || !q_b) return MRFG_ERR_ARG;

@@ -277,7 +277,7 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
         // only lets the first rounds run further ahead)
         const int window = max(2 * kHelpers, kWarmBytes / (V.lvWaves * 64 * (int)(sizeof(R) * G + sizeof(int) * K + sizeof(T))));
         for (int i = (int)blockIdx.x / kXcds - 1; i < g.nRounds; i += kHelpers) {
-            for (int spins = 0; spins < kPollLimit && i > __hip_atomic_load(&V.lvProgress[gi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + window; ++spins)
+            for (int spins = 0; spins < V.waitLimit && i > __hip_atomic_load(&V.lvProgress[gi], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + window; ++spins)
                 __builtin_amdgcn_s_sleep(8);
             Item S;
             load(i, roundOf(i), S);
@@ -521,7 +521,7 @@ __device__ __forceinline__ void boxFactor(const DiluView<double> &V, const int32
                     if (__builtin_amdgcn_ballot_w64(late) == 0) break;
                     // an expired wait ends every later one at once, so a
                     // broken schedule ends the kernel instead of hanging it
-                    if (spins >= kPollLimit || __hip_atomic_load(V.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                    if (spins >= V.waitLimit || __hip_atomic_load(V.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
                         if (lane == 0) atomicOr(V.err, 2);
                         break;
                     }

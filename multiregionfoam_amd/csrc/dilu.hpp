@@ -51,6 +51,8 @@ struct LevelGroup {
     int slice0, round0, nRounds, sys;
 };
 
+constexpr int kWaitLimit = 1 << 20;   // polls of one wait before it raises the error flag (about a second)
+
 template <typename T>
 struct DiluView {
     // chain waves in dispatch order
@@ -71,6 +73,7 @@ struct DiluView {
     double *rDout = nullptr;             // factor: plain rD per row
     const int32_t *cellOfPos = nullptr;  // factor: padding rows get rD = 0
     int *err = nullptr;                  // bit 2: a halo wait expired
+    int waitLimit = kWaitLimit;
     // structured-box tiles (dilu_box.hip; the factor in dilu.hip): their own
     // dispatch order, kBoxMeta ints of tile geometry per wave, and compact
     // inboxes of 2 max(TB, TC) values per step per tile, one per direction

@@ -215,9 +215,9 @@ __device__ __forceinline__ void boxCompute(const DiluView<T> &V, const int32_t *
             for (int spins = 0;; ++spins) {
                 lookReady();
                 if (isReady(need)) break;
-                // an expired wait ends every later one at once, so a broken
-                // schedule ends the kernel instead of hanging it
-                if ((spins & 1023) == 1023 && (spins > (kPollLimit << 3) || __hip_atomic_load(V.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
+                // an expired wait ends every later one after 1024 looks, so
+                // a broken schedule ends the kernel instead of hanging it
+                if ((spins & 1023) == 1023 && (spins > (kWaitLimit << 3) || __hip_atomic_load(V.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
                     if (lane == 0) atomicOr(V.err, 2);
                     break;
                 }
@@ -374,7 +374,7 @@ __device__ __forceinline__ void boxStream(const DiluView<T> &V, const Tile &t, S
             if (u % kChunk == 0) {
                 // room for the next chunk in the ring (bounded: the compute
                 // wave ends even if its waits expire)
-                for (int spins = 0; consumed + kRec < i + kChunk && spins < (kPollLimit << 4); ++spins) {
+                for (int spins = 0; consumed + kRec < i + kChunk && spins < (kWaitLimit << 4); ++spins) {
                     consumed = peek(&sh.consumed);
                     if (consumed + kRec < i + kChunk) __builtin_amdgcn_s_sleep(1);
                 }
@@ -465,11 +465,14 @@ __device__ __forceinline__ void boxFeed(const DiluView<T> &V, const int32_t *m, 
     };
 #pragma unroll
     for (int k = 0; k < kBatches; ++k) issue(ring[k]);
-    // (bounded: with a broken schedule every tile's feed wave gives up.  The
-    // loop has one exit, after whole rounds of batches: an exit in between
-    // made the compiler drain every load at the start of a round.)
+    // (bounded: `idle` rounds in a row without a step, not the rounds of a
+    // long sweep, and none once another wait has expired.  The loop has one
+    // exit, after whole rounds of batches: an exit in between made the
+    // compiler drain every load at the start of a round.)
     int done = 0;
-    for (int spins = 0; spins < kPollLimit && done != kAll; ++spins) {
+    for (int idle = 0; idle < V.waitLimit && done != kAll; ++idle) {
+        if (__builtin_expect((idle & 1023) == 1023, 0) && __hip_atomic_load(V.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            idle = V.waitLimit - 1;
 #pragma unroll
         for (int s = 0; s < kBatches; ++s) {
             Batch &q = ring[s];
@@ -500,6 +503,7 @@ __device__ __forceinline__ void boxFeed(const DiluView<T> &V, const int32_t *m, 
                 do done += kSub;
                 while (done < nL && __builtin_amdgcn_ballot_w64(lacks < done + kSub) == 0);
                 done = done < nL ? done : kAll;
+                idle = -1;
                 post(&sh.ready.edges, done);
             }
         }

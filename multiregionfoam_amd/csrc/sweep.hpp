@@ -7,8 +7,6 @@
 
 namespace mrfg {
 
-constexpr int kPollLimit = 1 << 20;   // polls of one wait before it raises the error flag
-
 template <typename T>
 struct Bits;
 template <>

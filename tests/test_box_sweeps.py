@@ -55,3 +55,43 @@ def test_sweeps_match_oracle(gpu, n):
     assert got.n_iterations == perf["nIterations"] and got.final_residual == perf["finalResidual"]
     assert np.array_equal(np.concatenate(A.psi(0)), np.concatenate(psi))
     A.close()
+
+
+def _committed(gpu, regions):
+    A = gpu.CoupledFvMatrix(0)
+    A.add_system(regions, [])
+    A.commit()
+    return A
+
+
+def test_wait_limit_is_of_one_wait(gpu):
+    # two flat tiles of 30000 steps: the second waits for a few steps of the
+    # first at a time, some 4000 polls in the whole sweep
+    regions = [box((30000, 66, 1), 4)]
+    A = _committed(gpu, regions)
+    assert len(set(A.dilu_tiles())) > 1
+    rD = A.dilu_factor()
+    r = [np.random.default_rng(5).standard_normal(R["nCells"]) for R in regions]
+    w = A.precondition(r)
+    A.set_wait_limit(500)
+    assert np.array_equal(A.dilu_factor(), rD)
+    assert np.array_equal(A.precondition(r), w)
+    A.close()
+
+
+def test_expired_wait_fails_the_call(gpu):
+    # a tile waits for its neighbour's first 64 steps: more than one poll
+    regions = [box((300, 130, 1), 6)]
+    A = _committed(gpu, regions)
+    A.dilu_factor()
+    r = [np.random.default_rng(7).standard_normal(R["nCells"]) for R in regions]
+    w = A.precondition(r)
+    A.set_wait_limit(1)
+    with pytest.raises(Exception, match="wait expired"):
+        A.precondition(r)
+    A.set_wait_limit(1 << 20)
+    assert np.array_equal(A.precondition(r), w)
+    for polls in (0, (1 << 20) + 1):
+        with pytest.raises(Exception, match="polls must be"):
+            A.set_wait_limit(polls)
+    A.close()
