@@ -823,6 +823,7 @@ void Batch::checkDeviceError()
     HIP_OK(hipStreamSynchronize(stream_));
     if (e) {
         err_.zero(stream_);
+        factorised_ = false;   // it may be the factor's
         throw std::runtime_error("HIP error: DILU dependency wait expired (device error flag " + std::to_string(e) +
                                  ")");
     }

@@ -87,10 +87,13 @@ def test_expired_wait_fails_the_call(gpu):
     r = [np.random.default_rng(7).standard_normal(R["nCells"]) for R in regions]
     w = A.precondition(r)
     A.set_wait_limit(1)
-    with pytest.raises(Exception, match="wait expired"):
-        A.precondition(r)
-    A.set_wait_limit(1 << 20)
-    assert np.array_equal(A.precondition(r), w)
+    # the sweep's wait, then the factor's, whose values must not be kept
+    for call in (lambda: A.precondition(r), A.dilu_factor):
+        with pytest.raises(Exception, match="wait expired"):
+            call()
+        A.set_wait_limit(1 << 20)
+        assert np.array_equal(A.precondition(r), w)
+        A.set_wait_limit(1)
     for polls in (0, (1 << 20) + 1):
         with pytest.raises(Exception, match="polls must be"):
             A.set_wait_limit(polls)
