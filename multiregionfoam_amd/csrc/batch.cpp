@@ -11,6 +11,7 @@
 #include <array>
 #include <chrono>
 #include <cstring>
+#include <map>
 #include <stdexcept>
 #include <thread>
 
@@ -32,6 +33,21 @@ std::recursive_mutex &deviceMutex()
 {
     static std::recursive_mutex m;
     return m;
+}
+
+// the gate of the current device's box sweeps (called under deviceMutex)
+static SweepGate &sweepGate(int device, int xcds)
+{
+    static std::map<int, std::unique_ptr<SweepGate>> gates;
+    std::unique_ptr<SweepGate> &g = gates[device];
+    if (!g) {
+        int perCU = 0;
+        HIP_OK(boxTilesPerCU(&perCU));
+        int cus = 0;
+        HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+        g.reset(new SweepGate(perCU * (cus / xcds)));
+    }
+    return *g;
 }
 
 template <typename T>
@@ -137,6 +153,10 @@ Batch::Batch(int device) : device_(device)
     HIP_OK(hipStreamCreateWithFlags(&side_, hipStreamNonBlocking));
     HIP_OK(hipEventCreateWithFlags(&fork_, hipEventDisableTiming));
     HIP_OK(hipEventCreateWithFlags(&join_, hipEventDisableTiming));
+    int cus = 0;
+    HIP_OK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device_));
+    xcds_ = xcdsOf(cus);
+    sweepGate_ = &sweepGate(device_, xcds_);
 }
 
 Batch::~Batch()
@@ -1128,6 +1148,7 @@ void Batch::solve(const SolverControls &c, std::vector<SolvePerf> &perf, const s
 {
     if (active && active->size() != sys_.size()) throw std::runtime_error("active mask does not match the batch");
     HIP_OK(hipSetDevice(device_));
+    const SweepHold hold(*sweepGate_, tilesPerXcd());
     struct ClearRetire {
         const RetireFn *&r;
         ~ClearRetire() { r = nullptr; }
@@ -1266,6 +1287,7 @@ void Batch::spmv(const double *xHost, double *yHost, int sys)
 
 void Batch::diluFactor(int sys, double *rDHost)
 {
+    const SweepHold hold(*sweepGate_, tilesPerXcd());
     applyRefresh();
     factorised_ = false;
     factorise();
@@ -1279,6 +1301,7 @@ void Batch::diluFactor(int sys, double *rDHost)
 
 void Batch::precondition(const double *rHost, double *wHost, int sys)
 {
+    const SweepHold hold(*sweepGate_, tilesPerXcd());
     applyRefresh();
     factorise();
     const SystemLayout &L = *lay_.at(sys);
@@ -1452,6 +1475,7 @@ void Batch::tilesOf(int sys, int *tileOfCell) const
 
 void Batch::precondition32(const float *rHost, float *wHost, int sys, bool tileLocal)
 {
+    const SweepHold hold(*sweepGate_, tilesPerXcd());
     applyRefresh();
     ensureFloat(tileLocal);
     factorise();
@@ -1479,6 +1503,7 @@ double Batch::timeKernel(int which, int reps)
     HIP_OK(hipSetDevice(device_));
     applyRefresh();
     if (which == 7 || which == 8) return timeAssembly(which, reps);
+    const SweepHold hold(*sweepGate_, tilesPerXcd());
     factorise();
     markAllRunning();
     Krylov<double> K;
@@ -1543,6 +1568,7 @@ double Batch::timeKernel(int which, int reps)
 int Batch::traceDilu(long long *out, int maxWaves)
 {
     HIP_OK(hipSetDevice(device_));
+    const SweepHold hold(*sweepGate_, tilesPerXcd());
     applyRefresh();
     factorise();
     markAllRunning();

@@ -24,6 +24,7 @@
 #include "dictionary.hpp"
 #include "kernels.hpp"
 #include "layout.hpp"
+#include "sweep_gate.hpp"
 
 namespace mrfg {
 
@@ -361,6 +362,9 @@ private:
     int nSlices_ = 0, nPos_ = 0, nBlk_ = 0, nWaves_ = 0, K_ = 3;
     int nGenWaves_ = 0, nBoxWaves_ = 0, nBoxIn_ = 0;
     int waitLimit_ = kWaitLimit;
+    SweepGate *sweepGate_ = nullptr;   // the device's
+    int tilesPerXcd() const { return boxLone_ ? 0 : (nBoxWaves_ + xcds_ - 1) / xcds_; }
+    int xcds_ = 1;
     bool boxLone_ = false;   // every box tile alone in its region
     bool factorised_ = false, haveFloat_ = false;
     bool tileLocal32_ = false;   // the FP32 records are those of the tile-local DILU

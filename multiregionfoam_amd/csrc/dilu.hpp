@@ -157,6 +157,13 @@ __host__ __device__ inline void boxSegment(int nA, int s, int segs, int &lo, int
     lo = (int)((long long)s * nA / segs);
     hi = (int)((long long)(s + 1) * nA / segs);
 }
+// Workgroups of the box sweeps (FP64, with inboxes) that a CU of the current
+// device holds at once
+hipError_t boxTilesPerCU(int *tiles);
+// XCDs of a device with `cus` CUs
+constexpr int kCusPerXcd = 32;
+inline int xcdsOf(int cus) { return cus > kCusPerXcd ? cus / kCusPerXcd : 1; }
+
 // Values of a box tile's inbox: per step one row for the b and one for the c edge
 __host__ __device__ inline int boxInboxValues(int nSteps, int TB) { return nSteps * 2 * (TB > 64 / TB ? TB : 64 / TB); }
 

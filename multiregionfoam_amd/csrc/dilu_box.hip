@@ -555,7 +555,8 @@ __device__ inline void initShared(Shared<T> &sh, bool fed)
 
 // One workgroup per tile (a LONE launch: per tile segment).  Workgroups are
 // dispatched in the order of their tiles' dependencies, so a tile only waits
-// for tiles that are resident or done.
+// for tiles that are resident or done (sweep_gate.hpp: also beside other
+// batches' sweeps).
 template <typename T, int KT, int MODE, bool LONE, int INP = kInpPlain>
 __global__ __launch_bounds__(LONE ? 128 : 192) void k_dilu_box(DiluView<T> V, const SysState *st, const T *in, T *out,
                                                                typename Bits<T>::U *inbox,
@@ -726,6 +727,21 @@ hipError_t diluApplyFused(const DiluView<T> &V, const SysState *st, int inp, con
     else k_dilu_box<T, 3, kDiluFwd, false, kInpS><<<n, 192, 0, s>>>(V, st, dst, out, use, clr, in);
     hipError_t e = hipGetLastError();
     return e != hipSuccess ? e : boxBackward<T>(V, st, out, s);
+}
+
+hipError_t boxTilesPerCU(int *tiles)
+{
+    const void *kernels[] = {(const void *)k_dilu_box<double, 3, kDiluBwd, false>, (const void *)k_dilu_box<double, 3, kDiluFwd, false, kInpP>,
+                             (const void *)k_dilu_box<double, 0, kDiluFwd, false>};
+    *tiles = INT_MAX;
+    for (const void *k : kernels) {
+        int n = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k, 192, 0);
+        if (e != hipSuccess) return e;
+        if (n < 1) return hipErrorInvalidValue;
+        *tiles = n < *tiles ? n : *tiles;
+    }
+    return hipSuccess;
 }
 
 #define MRFG_BOX_INSTANTIATE(T)                                                                                      \
