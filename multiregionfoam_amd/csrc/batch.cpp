@@ -84,6 +84,7 @@ template struct DevBuf<unsigned long long>;
 template struct DevBuf<int8_t>;
 template struct DevBuf<LevelGroup>;
 template struct DevBuf<LevelRound>;
+template struct DevBuf<SpreadSlice>;
 template struct DevBuf<FvRegionParams>;
 template struct DevBuf<DnaSide>;
 template struct DevBuf<DnaCell>;
@@ -292,7 +293,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     std::vector<unsigned long long> ifMask;
     std::vector<int32_t> cellOfPos, fCode, bCode, waveSlice, waveSteps, waveSys;
     std::vector<const std::vector<int32_t> *> waveLevels;
-    std::vector<uint8_t> waveFar;
+    std::vector<uint8_t> waveFar, waveSpread;
     std::vector<double> diag, source, sumA, psi0, fProd;
     std::vector<std::array<int, 3>> waveKey;   // (key, system, global wave index)
     std::vector<uint8_t> waveBox;
@@ -371,6 +372,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
             waveBox.push_back(L.waveBox[w]);
             waveLevels.push_back(&L.waveLevels[w]);
             waveFar.push_back(L.waveFar[w]);
+            waveSpread.push_back(L.waveSpread[w]);
             // box tile geometry with batch-wide wave, slice and inbox indices
             const int32_t *lm = &L.boxMeta[(size_t)w * kBoxMeta];
             std::array<int32_t, kBoxMeta> gm;
@@ -424,7 +426,8 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
                 }
                 prod[(((size_t)s * G + K_ / 2) * 64 + l) * 2 + K_ % 2] = diag[s * kSlice + l];
             }
-        // a chain's codes as bytes; a level group's as they are
+        // a chain's codes as bytes; a level group's as they are; spread levels'
+        // with batch-wide positions
         bool chains = false, groups = false;
         for (size_t w = 0; w < waveSlice.size(); ++w)
             if (!waveBox[w]) (waveLevels[w]->empty() ? chains : groups) = true;
@@ -447,6 +450,13 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
             }
             return v;
         };
+        for (size_t w = 0; w < waveSlice.size(); ++w) {
+            if (!waveSpread[w]) continue;
+            const size_t e1 = (size_t)(waveSlice[w] + waveSteps[w]) * K_ * kSlice;
+            for (size_t e = (size_t)waveSlice[w] * K_ * kSlice; e < e1; ++e)
+                for (std::vector<int32_t> *code : {&fCode, &bCode})
+                    if ((*code)[e] != kNoDep) (*code)[e] += waveSlice[w] * kSlice;
+        }
         fCodes_.upload(bytes(fCode), stream_);
         bCodes_.upload(bytes(bCode), stream_);
         fDeps_.upload(groups ? fCode : std::vector<int32_t>(1, kNoDep), stream_);
@@ -470,15 +480,15 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
     // forward dispatch order: by key (tile anti-diagonal), systems
     // interleaved; every tile's producers precede it.  Box tiles, chains and
     // level groups never depend on each other (DILU dependencies stay inside
-    // a region) and run in kernels of their own.
+    // a region) and run in kernels of their own; so do spread levels.
     std::sort(waveKey.begin(), waveKey.end());
     std::vector<int32_t> order, boxOrder;
-    std::vector<int> grouped;
+    std::vector<int> grouped, spreadOut;
     for (int i = 0; i < nWaves_; ++i) {
         const int w = waveKey[i][2];
         if (waveBox[w]) boxOrder.push_back(w);
         else if (waveLevels[w]->empty()) order.push_back(w);
-        else grouped.push_back(w);
+        else (waveSpread[w] ? spreadOut : grouped).push_back(w);
     }
     // level groups: rounds of as many slices of one level as a workgroup has
     // waves (as many as the widest level needs, at most 16)
@@ -495,6 +505,24 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
         groups.push_back(g);
     }
     nGroups_ = (int)groups.size();
+    std::vector<std::vector<SpreadSlice>> byLevel;
+    for (size_t r = 0; r < spreadOut.size(); ++r) {
+        const int w = spreadOut[r];
+        const std::vector<int32_t> &levels = *waveLevels[w];
+        if (byLevel.size() < levels.size()) byLevel.resize(levels.size());
+        int s = waveSlice[w];
+        for (size_t lv = 0; lv < levels.size(); ++lv)
+            for (int k = 0; k < levels[lv]; ++k, ++s)
+                byLevel[lv].push_back({s, waveSys[w], (int)r, k == 0 ? (int)levels.size() : 0});
+    }
+    std::vector<SpreadSlice> spread;
+    spreadLevels_.assign(1, 0);
+    for (const auto &lv : byLevel) {
+        spread.insert(spread.end(), lv.begin(), lv.end());
+        spreadLevels_.push_back((int)spread.size());
+    }
+    if (spread.empty()) spread.push_back(SpreadSlice{});
+    spread_.upload(spread, stream_);
     if (groups.empty()) groups.push_back(LevelGroup{});
     if (rounds.empty()) rounds.push_back(LevelRound{0, 0});
     groups_.upload(groups, stream_);
@@ -717,6 +745,9 @@ DiluView<T> Batch::diluView(DevMatrix<T> &m, void *hF, void *hB)
     D.nGroups = nGroups_;
     D.lvWaves = lvWaves_;
     D.lvD = lvD_.p;
+    D.spread = spread_.p;
+    D.spreadLevels = spreadLevels_.data();
+    D.nSpreadLevels = (int)spreadLevels_.size() - 1;
     D.lvProgress = lvProgress_.p;
     D.boxInF = hF;
     D.boxInB = hB;

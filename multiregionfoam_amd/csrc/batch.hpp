@@ -409,6 +409,8 @@ private:
     DevBuf<LevelRound> lvRounds_;
     DevBuf<double> lvD_;                          // d of the level groups' rows (factor)
     int nGroups_ = 0, lvWaves_ = 1;
+    DevBuf<SpreadSlice> spread_;
+    std::vector<int> spreadLevels_;               // first slice of each level in spread_, then the end
     DevBuf<double2> prodPack_;
     DevBuf<unsigned long long> haloF64_, haloB64_, haloC64_;
     DevBuf<unsigned int> haloF32_, haloB32_;

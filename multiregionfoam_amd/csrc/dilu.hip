@@ -375,6 +375,69 @@ __global__ __launch_bounds__(1024) void k_dilu_levels(DiluView<T> V, const SysSt
     }
 }
 
+// Spread levels: one launch per level, a wave per slice over the whole device,
+// every dependency read from memory.  Bound by the launches (3.6 us each in a
+// graph) up to some 10^4 rows a level, above by the reads of rows spread over
+// memory: 170 us a sweep for 2.0M shuffled cells in 24 levels, where one
+// workgroup takes 8300 us and a wave per slice that polls for its dependencies
+// took 4500.  No workgroup waits for another.
+template <typename T, int K, int MODE>
+__global__ __launch_bounds__(256) void k_dilu_spread(DiluView<T> V, const SysState *st, const T *in, T *out, int first,
+                                                     int n)
+{
+    using R = typename RecordOf<T, MODE>::V;
+    constexpr int N = RecordOf<T, MODE>::N;
+    constexpr int G = packChunks(K + 1, N);
+    const int i = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= n) return;
+    const SpreadSlice q = V.spread[first + i];
+    if (MODE != kDiluFactor && st[q.sys].status != kRunning) return;
+    const unsigned long long tStart = V.trace ? wall_clock64() : 0ull;
+    const int32_t *deps = MODE == kDiluBwd ? V.bDeps : V.fDeps;
+    const R *recs = MODE == kDiluFactor ? (const R *)V.prodPack : (const R *)(MODE == kDiluBwd ? V.bPack : V.fPack);
+    const size_t s = (size_t)q.slice, p = s * 64 + lane;
+    int c[K];
+    R v[G];
+    T a = T(0), x[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) c[k] = deps[(s * K + k) * 64 + lane];
+#pragma unroll
+    for (int g = 0; g < G; ++g) v[g] = recs[(s * G + g) * 64 + lane];
+    if (MODE != kDiluFactor) a = in[p];
+    // (stored by an earlier launch)
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const size_t from = c[k] == kNoDep ? p : (size_t)c[k];
+        x[k] = MODE == kDiluFactor ? (T)V.lvD[from] : out[from];
+    }
+    const T last = (T)elem(v[K / N], K % N);   // rD, or diag for the factor
+    T y = MODE == kDiluFwd ? a * last : MODE == kDiluBwd ? a : last;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const T f = (T)elem(v[k / N], k % N);
+        const T t = MODE == kDiluFactor ? y - f / x[k] : y - last * f * x[k];
+        y = c[k] != kNoDep ? t : y;
+    }
+    if (MODE == kDiluFactor) {
+        const double rd = V.cellOfPos[p] >= 0 ? 1.0 / (double)y : 0.0;
+        V.rDout[p] = rd;
+        V.lvD[p] = (double)y;
+        constexpr int NP = Pack<double>::N;
+        constexpr int GP = packChunks(K + 1, NP);
+        ((double *)&V.fPack[(s * GP + K / NP) * 64 + lane])[K % NP] = rd;
+        ((double *)&V.bPack[(s * GP + K / NP) * 64 + lane])[K % NP] = rd;
+    } else {
+        out[p] = y;
+    }
+    if (V.trace && q.levels && lane == 0) {
+        unsigned long long *tr = V.trace + 4 * ((size_t)V.nWaves + V.nBoxWaves + V.nGroups + q.region);
+        if (tr[0] == 0) tr[0] = tStart;
+        tr[1] = wall_clock64();
+        tr[2] = 0;
+        tr[3] = (unsigned long long)q.levels;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Factorisation of structured-box tiles (the sweeps are in dilu_box.hip).
 //
@@ -602,12 +665,17 @@ static void launchGeneralK(const DiluView<T> &V, const SysState *st, const T *in
         const int blocks = L.lvHelped ? kXcds * (1 + kHelpers) : V.nGroups;
         k_dilu_levels<T, K, MODE><<<blocks, 64 * V.lvWaves, 0, s>>>(L, st, in, out);
     }
+    for (int i = 0; i < V.nSpreadLevels; ++i) {
+        const int lv = MODE == kDiluBwd ? V.nSpreadLevels - 1 - i : i;
+        const int first = V.spreadLevels[lv], n = V.spreadLevels[lv + 1] - first;
+        k_dilu_spread<T, K, MODE><<<(n + 3) / 4, 256, 0, s>>>(V, st, in, out, first, n);
+    }
 }
 
 template <typename T, int MODE>
 static hipError_t launchGeneral(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s)
 {
-    if (V.nWaves <= 0 && V.nGroups <= 0) return hipSuccess;
+    if (!V.general()) return hipSuccess;
     if (V.lvWaves < 1 || V.lvWaves > 16) return hipErrorInvalidValue;
     switch (V.K) {
     case 3: launchGeneralK<T, 3, MODE>(V, st, in, out, s); break;
@@ -640,7 +708,7 @@ static hipError_t launchBoxFactor(const DiluView<double> &V, hipStream_t s)
 template <typename T, typename GenF, typename BoxF>
 static hipError_t bothSweeps(const DiluView<T> &V, hipStream_t s, GenF &&gen, BoxF &&box)
 {
-    const bool fork = V.side && V.fork && V.join && V.nWaves + V.nGroups > 0 && V.nBoxWaves > 0;
+    const bool fork = V.side && V.fork && V.join && V.general() && V.nBoxWaves > 0;
     if (!fork) {
         hipError_t e = gen(s);
         return e != hipSuccess ? e : box(s);

@@ -29,7 +29,7 @@ constexpr unsigned int kHaloSentinel32 = 0xFFA5A5A5u;
 //                 int, int j of lane l of slice s at (s*NC + j)*64 + l;
 //   level groups  one int each, that of slot k at (s*K + k)*64 + l: kNoDep,
 //                 an LDS ring slot (< kLevelRing), or kLevelRing + the row's
-//                 place in the group.
+//                 place in the group; spread levels: the row's position.
 template <typename T>
 struct Pack;
 template <>
@@ -53,6 +53,13 @@ struct LevelGroup {
 
 constexpr int kWaitLimit = 1 << 20;   // polls of one wait before it raises the error flag (about a second)
 
+// A slice of a region whose levels are spread over the device
+struct SpreadSlice {
+    int slice, sys;
+    int region;      // among the spread regions
+    int levels;      // of the region, in the first slice of a level; else 0
+};
+
 template <typename T>
 struct DiluView {
     // chain waves in dispatch order
@@ -67,11 +74,17 @@ struct DiluView {
     int nGroups = 0, lvWaves = 1;
     int *lvProgress = nullptr;           // per group: the round its sweep has reached
     bool lvHelped = false;               // set by the launcher: helper workgroups read lvProgress
-    double *lvD = nullptr;               // factor: d per row of the level groups
+    double *lvD = nullptr;               // factor: d per row of the level groups and spread levels
+    // spread levels: the slices of all regions' first level, of their second
+    // and so on; level l has those from spreadLevels[l] on (on the host)
+    const SpreadSlice *spread = nullptr;
+    const int *spreadLevels = nullptr;
+    int nSpreadLevels = 0;
     typename Pack<T>::V *fPack = nullptr, *bPack = nullptr;
     const double2 *prodPack = nullptr;   // factor records (FP64)
     double *rDout = nullptr;             // factor: plain rD per row
     const int32_t *cellOfPos = nullptr;  // factor: padding rows get rD = 0
+    bool general() const { return nWaves > 0 || nGroups > 0 || nSpreadLevels > 0; }   // regions that are no boxes
     int *err = nullptr;                  // bit 2: a halo wait expired
     int waitLimit = kWaitLimit;
     // structured-box tiles (dilu_box.hip; the factor in dilu.hip): their own
@@ -91,7 +104,7 @@ struct DiluView {
     int nBoxIn = 0;
     // optional trace: per wave start / end realtime clock ticks, slow-path
     // hits and steps (4 entries each); chain waves by dispatch index, then box
-    // tiles, then level groups
+    // tiles, then level groups, then spread regions
     unsigned long long *trace = nullptr;
     // host side: when both kinds of waves exist, the box sweep runs on `side`
     // concurrently with the general sweep (regions never depend on each
@@ -140,7 +153,7 @@ hipError_t diluApplyFused(const DiluView<T> &V, const SysState *st, int inp, con
 template <typename T>
 bool diluCanFuse(const DiluView<T> &V)
 {
-    return V.nWaves == 0 && V.nGroups == 0 && V.nBoxWaves > 0 && V.K == 3;
+    return !V.general() && V.nBoxWaves > 0 && V.K == 3;
 }
 // Factorisation: rD = 1/d for every row of the batch (FP64), written to
 // rDout and into the forward and backward records.

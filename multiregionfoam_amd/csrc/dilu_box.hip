@@ -698,7 +698,7 @@ hipError_t boxBackward(const DiluView<T> &V, const SysState *st, T *inout, hipSt
 template <typename T>
 hipError_t diluApplyLone(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s)
 {
-    if (V.nBoxWaves <= 0 || V.nWaves > 0 || V.nGroups > 0 || !V.boxLone || !V.boxTile) return hipErrorInvalidValue;
+    if (V.nBoxWaves <= 0 || V.general() || !V.boxLone || !V.boxTile) return hipErrorInvalidValue;
     const int nb = V.nBoxWaves * (V.boxSegs > 1 ? V.boxSegs : 1);
     if (V.K == 3) k_dilu_box_pair<T, 3><<<nb, 128, 0, s>>>(V, st, in, out);
     else k_dilu_box_pair<T, 0><<<nb, 128, 0, s>>>(V, st, in, out);

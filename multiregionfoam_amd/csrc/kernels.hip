@@ -646,7 +646,7 @@ hipError_t launchSetup(const MatView<T> &A, const Krylov<T> &K, bool pcg, hipStr
 template <typename T>
 hipError_t launchPrecondition(const DiluView<T> &D, const Krylov<T> &K, const T *in, T *out, hipStream_t st)
 {
-    if (D.boxLone && D.nWaves == 0 && D.nGroups == 0 && D.nBoxWaves > 0) return diluApplyLone<T>(D, K.state, in, out, st);
+    if (D.boxLone && !D.general() && D.nBoxWaves > 0) return diluApplyLone<T>(D, K.state, in, out, st);
     hipError_t e = diluForward<T>(D, K.state, in, out, st);
     if (e != hipSuccess) return e;
     return diluBackward<T>(D, K.state, out, st);

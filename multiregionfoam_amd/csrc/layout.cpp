@@ -23,7 +23,8 @@ struct WaveBuild {
     // structured-box tile (box = false for level waves)
     bool box = false;
     int tb = 0, tc = 0, TB = 0, nA = 0, seqAxis = 0, actB = 0, actC = 0;
-    std::vector<int32_t> levels;   // level group: slices per level
+    std::vector<int32_t> levels;   // level group or spread levels: slices per level
+    bool spread = false;
 };
 
 void tangential(int a, int &b, int &c)
@@ -108,6 +109,46 @@ void boxWaves(const int n[3], int regionIdx, int cellOffset, RegionSchedule &rs,
         }
 }
 
+// Whether a region's levels are swept by the whole device, one launch per
+// level, rather than by one workgroup (a level group).  What a sweep takes
+// (FP64, launches replayed from a graph):
+//   spread   3.6 us a level (1340 us for 382 levels of 2.0M cells numbered
+//            along a front, 170 us for 20 levels of 2.0M shuffled cells)
+//   group    0.8 ns a row (389 us for 0.5M cells along a front, 241 levels),
+//            and 1.1 ns for each line of 128 bytes that a slice reads back
+//            from beyond the LDS ring (2030 us for the 2.0M along a front,
+//            1960 us for 0.5M shuffled, 8300 us for 2.0M shuffled)
+// so a level is worth 4500 rows and such a line 1.5.  The other choice: spread
+// 870 us for the 0.5M along a front, 1180 (against 967) for 1.3M in 328
+// levels; a group 143 us (against 61) for 59k shuffled cells in 17 levels.
+bool spreadPays(int c0, int c1, const RowDeps &D, const std::vector<std::vector<int32_t>> &byLevel)
+{
+    constexpr long long kRowsPerLevel = 4500;
+    constexpr int kLine = 128 / sizeof(double);
+    const long long rows = c1 - c0, need = kRowsPerLevel * (long long)byLevel.size();
+    if (rows >= need) return true;
+    std::vector<int32_t> place(c1 - c0);   // in the group's slices
+    int32_t at = 0;
+    long long lines = 0;
+    std::vector<int32_t> back;             // lines of a slice
+    for (const std::vector<int32_t> &cells : byLevel) {
+        const int32_t end = at + (int32_t)((cells.size() + kSlice - 1) / kSlice) * kSlice;
+        for (size_t i = 0; i < cells.size(); ++i) place[cells[i] - c0] = at + (int32_t)i;
+        for (size_t i = 0; i < cells.size(); i += kSlice) {
+            back.clear();
+            for (size_t l = i; l < std::min(i + kSlice, cells.size()); ++l)
+                for (int q = D.lo_off[cells[l]]; q < D.lo_off[cells[l] + 1]; ++q) {
+                    const int32_t from = place[D.lo_nb[q] - c0];
+                    if (end - from > kLevelRing) back.push_back(from / kLine);
+                }
+            std::sort(back.begin(), back.end());
+            lines += std::unique(back.begin(), back.end()) - back.begin();
+        }
+        at = end;
+    }
+    return 2 * rows + 3 * lines >= 2 * need;
+}
+
 void levelWaves(int regionIdx, int c0, int c1, const RowDeps &D, RegionSchedule &rs, std::vector<WaveBuild> &out)
 {
     std::vector<int32_t> level(c1 - c0, 0);
@@ -131,7 +172,7 @@ void levelWaves(int regionIdx, int c0, int c1, const RowDeps &D, RegionSchedule 
     // one wave walks narrow levels as its steps: every dependency comes from
     // its own LDS ring and no step waits for another wave.  Wider levels (or
     // levels that reach further back) go to a workgroup with a barrier per
-    // level.
+    // level, or are spread over the device where they are wide enough.
     const bool chain = maxWidth <= (size_t)kSlice && reach <= kRing - 1;
     for (int lv = 0; lv <= maxLevel; ++lv) {
         const int n = (int)((byLevel[lv].size() + kSlice - 1) / kSlice);
@@ -141,7 +182,8 @@ void levelWaves(int regionIdx, int c0, int c1, const RowDeps &D, RegionSchedule 
         if (!chain) w.levels.push_back(n);
         w.steps += n;
     }
-    rs.kind = chain ? "chain" : "levels";
+    w.spread = !chain && spreadPays(c0, c1, D, byLevel);
+    rs.kind = chain ? "chain" : w.spread ? "spread" : "levels";
     rs.nWaves = 1;
     rs.maxSteps = w.steps;
     out.push_back(std::move(w));
@@ -288,6 +330,7 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
     L.waveKey.resize(L.nWaves);
     L.waveLevels.resize(L.nWaves);
     L.waveFar.assign(L.nWaves, 0);
+    L.waveSpread.assign(L.nWaves, 0);
     int slice = 0;
     for (int wi = 0; wi < L.nWaves; ++wi) {
         const WaveBuild &w = waves[ord[wi]];
@@ -295,6 +338,7 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
         L.waveSteps[wi] = w.steps;
         L.waveKey[wi] = w.key;
         L.waveLevels[wi] = w.levels;
+        L.waveSpread[wi] = w.spread ? 1 : 0;
         slice += w.steps;
     }
     L.nSlices = slice;
@@ -569,8 +613,8 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
                         if (lvEnd[pd / kSlice] > lvBegin[s]) throw std::runtime_error("DILU schedule violates a forward dependency");
                         // in the ring until the rows kLevelRing further on are written
                         const int at = td * kSlice + ld;
-                        const bool far = lvEnd[s] * kSlice - at > kLevelRing;
-                        L.fCode[e] = far ? kLevelRing + at : at & (kLevelRing - 1);
+                        const bool far = !L.waveSpread[w] && lvEnd[s] * kSlice - at > kLevelRing;
+                        L.fCode[e] = L.waveSpread[w] ? at : far ? kLevelRing + at : at & (kLevelRing - 1);
                         if (far) L.waveFar[w] = 1;
                     } else {
                         if (t - td < 1 || t - td > kRing - 1) throw std::runtime_error("DILU schedule violates a forward dependency");
@@ -591,8 +635,8 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
                     if (lvEnd[s] >= 0) {
                         if (lvBegin[pd / kSlice] < lvEnd[s]) throw std::runtime_error("DILU schedule violates a backward dependency");
                         const int at = td * kSlice + ld;
-                        const bool far = at - lvBegin[s] * kSlice >= kLevelRing;
-                        L.bCode[e] = far ? kLevelRing + at : at & (kLevelRing - 1);
+                        const bool far = !L.waveSpread[w] && at - lvBegin[s] * kSlice >= kLevelRing;
+                        L.bCode[e] = L.waveSpread[w] ? at : far ? kLevelRing + at : at & (kLevelRing - 1);
                         if (far) L.waveFar[w] = 1;
                     } else {
                         if (td - t < 1 || td - t > kRing - 1) throw std::runtime_error("DILU schedule violates a backward dependency");

@@ -15,14 +15,15 @@
 //     the levels, where every level fits 64 rows and reaches at most
 //     kRing - 1 levels back (2-D and multi-block meshes, whose levels are
 //     anti-diagonals), else a level group, swept by one workgroup that meets
-//     at a barrier after each level.
+//     at a barrier after each level, or spread levels, each swept by the whole
+//     device, where they are wide.
 //
 // Either way the schedule is a topological order of the factor's dependency
 // graph, so the Cholesky/DILU factor and sweeps computed in it are the
 // reference preconditioner itself.  A chain's wave reads its dependencies
 // from an LDS ring of its last kRing steps, a level group from an LDS ring of
 // the region's last kLevelRing rows, or from memory where they lie further
-// back.
+// back, spread levels from memory.
 //
 // Per slice of 64 rows:
 //   SpMV   sliced ELL, column-major inside the slice: entry k of lane l at
@@ -36,7 +37,7 @@
 //          products, backward = upper neighbours in reverse face order with
 //          upper coefficients; codes: kNoDep, in a chain the ring slot, in a
 //          level group the ring slot or kLevelRing + the row's place in the
-//          region's slices.
+//          region's slices, in spread levels that place.
 #pragma once
 
 #include "coupled_system.hpp"
@@ -92,7 +93,7 @@ enum {
 enum { kSgAxis = 0, kSgLogTB, kSgPrevB, kSgNextB, kSgPrevC, kSgNextC, kSliceGeom = 8 };
 
 struct RegionSchedule {
-    std::string kind;                // "box", "chain" or "levels"
+    std::string kind;                // "box", "chain", "levels" or "spread"
     int n[3] = {0, 0, 0};            // box dimensions
     int seqAxis = -1, tileB = 0, tileC = 0;
     int nWaves = 0, maxSteps = 0;
@@ -128,9 +129,11 @@ struct SystemLayout {
     // DILU
     std::vector<int32_t> fCode, bCode;       // nSlices * K * 64
     std::vector<double> fVal, fProd, bVal;
-    // per wave: the slices of each level of a level group (empty for others)
+    // per wave: the slices of each level of a level group or of spread levels
+    // (empty for others)
     std::vector<std::vector<int32_t>> waveLevels;
     std::vector<uint8_t> waveFar;            // per wave: 1 if a dependency lies beyond the LDS ring
+    std::vector<uint8_t> waveSpread;         // per wave: 1 if its levels are spread over the device
     // structured-box tile waves: their rows keep the DILU values in fixed
     // slots (slot = 2 - axis of the neighbour: z, y, x, which is both the
     // face order of the lower neighbours and the reverse face order of the

@@ -12,7 +12,8 @@
 using namespace mrfg;
 
 // noWaits: the schedule without barriers that wait for stores;
-// out: ring reads, far reads, barriers, barriers that wait for stores
+// out: ring reads, far reads, barriers, barriers that wait for stores, reads of
+// spread levels
 extern "C" int replay(int nCells, int nFaces, const int32_t *lower, const int32_t *upper, int waves, int noWaits,
                       long long *out, char *why, int nWhy)
 try {
@@ -27,7 +28,8 @@ try {
     R.upper = R.lower;
     R.diag = R.source = R.psi = std::vector<double>(nCells, 1.0);
     const SystemLayout L = buildLayout(sys);
-    if (L.schedules[0].kind != "levels" || L.nWaves != 1) throw std::runtime_error("not a level group: " + L.schedules[0].kind);
+    const bool spread = L.schedules[0].kind == "spread";
+    if (!spread && L.schedules[0].kind != "levels") throw std::runtime_error("no levels: " + L.schedules[0].kind);
     std::vector<LevelRound> rounds;
     levelRounds(L.waveLevels[0], 0, waves, L.waveFar[0] != 0 && !noWaits, rounds);
     // neighbours in the order of the dependency slots
@@ -40,7 +42,28 @@ try {
         std::snprintf(why, nWhy, "%s at cell %d", what, cell);
         return 1;
     };
-    std::memset(out, 0, 4 * sizeof(long long));
+    std::memset(out, 0, 5 * sizeof(long long));
+    if (spread != (L.waveSpread[0] != 0)) return fail("wrong kind of wave", -1);
+    if (spread) {
+        std::vector<int> levelOf(L.nSlices);
+        int s = 0;
+        for (size_t lv = 0; lv < L.waveLevels[0].size(); ++lv)
+            for (int k = 0; k < L.waveLevels[0][lv]; ++k) levelOf[s++] = (int)lv;
+        if (s != L.nSlices) return fail("slice left out", -1);
+        for (int c = 0; c < nCells; ++c)
+            for (bool fwd : {true, false})
+                for (int k = 0; k < L.K; ++k) {
+                    const std::vector<int> &nb = fwd ? lo[c] : up[c];
+                    const int p = L.posOfCell[c], q = (fwd ? L.fCode : L.bCode)[((size_t)(p / kSlice) * L.K + k) * kSlice + p % kSlice];
+                    if ((q == kNoDep) != (k >= (int)nb.size())) return fail("wrong number of dependencies", c);
+                    if (q == kNoDep) continue;
+                    ++out[4];
+                    if (q != L.posOfCell[nb[k]]) return fail("wrong row", c);
+                    const int from = levelOf[q / kSlice], to = levelOf[p / kSlice];
+                    if (fwd ? from >= to : from <= to) return fail("row of a level launched later", c);
+                }
+        return 0;
+    }
     for (bool fwd : {true, false}) {
         enum { kNone, kWritten, kInMemory };
         std::vector<int> ring(kLevelRing, -1), state(L.nPos, kNone), seen(L.nSlices, 0), level;

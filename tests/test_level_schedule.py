@@ -1,6 +1,7 @@
-"""Host replay of the level groups' schedule: every dependency is in the LDS
-ring, or in memory behind a barrier that waits for stores, before its reader's
-level starts (tests/schedule_replay.cpp)."""
+"""Host replay of the schedule of regions on levels: every dependency is in a
+level group's LDS ring, or in memory behind a barrier that waits for stores,
+before its reader's level starts; in spread levels it is a row of a level
+launched before (tests/schedule_replay.cpp)."""
 import ctypes as C
 import os
 import subprocess
@@ -13,10 +14,6 @@ import test_level_sweeps as ls
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "multiregionfoam_amd", "csrc")
 
-CASES = dict({name: ls.CASES[name] for name in ls.CASES if name != "with_chain_and_box"},
-             several_narrow_then_wide=lambda: [ls.ladder(
-    [900] * 25 + [30] * 40 + [150, 800, 4000, 9000] + [100] * 30 + [500, 2500, 9500, 500])])
-
 
 @pytest.fixture(scope="module")
 def lib(tmp_path_factory):
@@ -27,18 +24,24 @@ def lib(tmp_path_factory):
 
 
 def replay(lib, R, waves, no_waits=0):
-    out, why = (C.c_longlong * 4)(), C.create_string_buffer(200)
+    out, why = (C.c_longlong * 5)(), C.create_string_buffer(200)
     p = lambda a: a.ctypes.data_as(C.POINTER(C.c_int32))  # noqa: E731
     rc = lib.replay(R["nCells"], R["nFaces"], p(R["lAddr"]), p(R["uAddr"]), waves, no_waits, out, why, len(why))
-    return rc, why.value.decode(), dict(zip(("ring", "far", "barriers", "stored"), out))
+    return rc, why.value.decode(), dict(zip(("ring", "far", "barriers", "stored", "spread"), out))
 
 
 @pytest.mark.parametrize("waves", [1, 3, 16])
-@pytest.mark.parametrize("name", list(CASES))
+@pytest.mark.parametrize("name", list(ls.CASES))
 def test_dependencies_are_where_their_codes_say(lib, name, waves):
-    for R in CASES[name]():
+    regions = ls.CASES[name]()
+    kinds = ls.KINDS.get(name, ["levels"] * len(regions))
+    for R, kind in zip(regions, kinds):
         rc, why, n = replay(lib, R, waves)
+        if kind not in ("levels", "spread"):
+            assert rc == 2 and why == "no levels: " + kind
+            continue
         assert rc == 0, why
+        assert (n["spread"] > 0) == (kind == "spread")
         # barriers that wait for stores: none without far rows, and no more
         # than two for each ring of rows in either direction (or one a level)
         rows = 64 * -(-R["nCells"] // 64) + 64 * n["barriers"] // 2

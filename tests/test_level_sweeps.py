@@ -75,6 +75,21 @@ def ladder(widths, seed=8):
                 diag=diag, source=rng.standard_normal(N), psi=rng.standard_normal(N))
 
 
+def layers(width, n, most):
+    """n levels of `width` cells, each cell with `most` lower neighbours in
+    the level before."""
+    c = np.arange(width)
+    f = np.concatenate([np.stack([(lv - 1) * width + (c + 7 * j) % width, lv * width + c], axis=1)
+                        for lv in range(1, n) for j in range(most)])
+    f = f[np.lexsort((f[:, 1], f[:, 0]))].astype(np.int32)
+    rng = np.random.default_rng(9)
+    u, lo = -rng.uniform(0.1, 1.0, len(f)), -rng.uniform(0.1, 1.0, len(f))
+    N = n * width
+    diag = 0.5 - np.bincount(f[:, 0], u, N) - np.bincount(f[:, 1], lo, N)
+    return dict(nCells=N, nFaces=len(f), symmetric=False, lAddr=f[:, 0].copy(), uAddr=f[:, 1].copy(), lower=lo, upper=u,
+                diag=diag, source=rng.standard_normal(N), psi=rng.standard_normal(N))
+
+
 def strip():
     """Three blocks side by side, numbered one after the other: a chain."""
     n = (60, 20, 1)
@@ -84,6 +99,11 @@ def strip():
     return renumbered(box(n, 7), b * 400 + j * 20 + i % 20)
 
 
+WIDE_AMONG_NARROW = [900] * 25 + [30] * 40 + [150, 800, 4000, 9000] + [100] * 30 + [500, 2500, 9500, 500]
+KINDS = {"beyond_the_ring": ["spread"], "spread_levels": ["spread", "spread"], "spread_twelve_neighbours": ["spread"],
+         "spread_beside_others": ["spread", "chain", "box", "levels", "spread"],
+         "with_chain_and_box": ["chain", "box", "levels"]}   # of the regions, if not all level groups
+
 CASES = {
     "narrow_levels": lambda: [front((23, 11, 9), 0.9)],
     "levels_over_a_workgroup": lambda: [front((60, 45, 40), 0.5), front((40, 33, 9), 2.5)],
@@ -91,6 +111,12 @@ CASES = {
     # a wide level, then levels that most waves of the workgroup have no part
     # in, with rows read back long after they have left the ring
     "far_rows_of_narrow_levels": lambda: [ladder([1000] + [300] * 110), ladder([2000, 700] + [64] * 300 + [300] + [900] * 5)],
+    "wide_among_narrow_levels": lambda: [ladder(WIDE_AMONG_NARROW)],
+    # spread over the device: a level of a few slices, of one row, of many
+    "spread_levels": lambda: [layers(6000, 4, 3), ladder([5000, 5000, 1, 5, 25, 125, 600, 3000, 15000, 17001])],
+    "spread_twelve_neighbours": lambda: [layers(5000, 3, 12)],
+    "spread_beside_others": lambda: [shuffled((40, 40, 30)), strip(), box((30, 17, 15), 8), front((12, 12, 12), 0.9),
+                                     layers(6000, 5, 2)],
     "six_neighbours": lambda: [shuffled((13, 11, 7))],
     "twelve_neighbours": lambda: [graph(1500, 12), front((17, 9, 8), 0.5)],
     "with_chain_and_box": lambda: [strip(), box((30, 17, 5), 8), front((12, 12, 12), 0.9)],
@@ -117,4 +143,8 @@ def test_level_sweeps_match_oracle(gpu, name):
     got = A.solve(tolerance=1e-10, maxIter=30)[0]
     assert got.n_iterations == perf["nIterations"]
     assert np.array_equal(np.concatenate(A.psi(0)), np.concatenate(psi))
+    # every wave, tile, group and spread region appears in the trace of both sweeps
+    for sweep in A.trace_dilu():
+        assert len(sweep) == A.layout_info(0)["waves"]
+        assert np.all(sweep[:, 1] >= sweep[:, 0]) and np.all(sweep[:, 0] >= 0) and np.all(sweep[:, 3] > 0)
     A.close()
