@@ -629,7 +629,7 @@ __global__ __launch_bounds__(LONE ? 128 : 192) void k_dilu_box(DiluView<T> V, co
 // Both sweeps of lone tiles in one launch: a workgroup sweeps its tile (or
 // tile segment) forward and then backward, since its backward rows depend
 // only on its own forward rows.
-template <typename T, int KT, int INP = kInpPlain>
+template <typename T, int INP = kInpPlain>
 __global__ __launch_bounds__(128) void k_dilu_box_pair(DiluView<T> V, const SysState *st, const T *in, T *out,
                                                        SweepInput<T> inpBase = SweepInput<T>{})
 {
@@ -648,7 +648,7 @@ __global__ __launch_bounds__(128) void k_dilu_box_pair(DiluView<T> V, const SysS
     initShared(sh, false);
     __syncthreads();
     if (wave == 0) computeAll<T, kDiluFwd, true>(V, m, t, sp, out, (U *)nullptr, sh, nSlow);
-    else boxStream<T, KT, kDiluFwd, INP>(V, t, sp, in, sh, INP ? sweepInputOf(INP, inpBase, st[m[kBtSys]]) : inpBase);
+    else boxStream<T, 3, kDiluFwd, INP>(V, t, sp, in, sh, INP ? sweepInputOf(INP, inpBase, st[m[kBtSys]]) : inpBase);
     // the forward rows of the compute wave are read back by the stream wave
     // (of the same workgroup)
     __builtin_amdgcn_s_waitcnt(0);
@@ -656,7 +656,7 @@ __global__ __launch_bounds__(128) void k_dilu_box_pair(DiluView<T> V, const SysS
     initShared(sh, false);
     __syncthreads();
     if (wave == 0) computeAll<T, kDiluBwd, true>(V, m, t, sp, out, (U *)nullptr, sh, nSlow);
-    else boxStream<T, KT, kDiluBwd, kInpPlain>(V, t, sp, out, sh, SweepInput<T>{});
+    else boxStream<T, 3, kDiluBwd, kInpPlain>(V, t, sp, out, sh, SweepInput<T>{});
 }
 
 // ---------------------------------------------------------------------------
@@ -698,10 +698,10 @@ hipError_t boxBackward(const DiluView<T> &V, const SysState *st, T *inout, hipSt
 template <typename T>
 hipError_t diluApplyLone(const DiluView<T> &V, const SysState *st, const T *in, T *out, hipStream_t s)
 {
-    if (V.nBoxWaves <= 0 || V.general() || !V.boxLone || !V.boxTile) return hipErrorInvalidValue;
+    // (records are wider than a box's three slots only beside other regions)
+    if (V.nBoxWaves <= 0 || V.general() || V.K != 3 || !V.boxLone || !V.boxTile) return hipErrorInvalidValue;
     const int nb = V.nBoxWaves * (V.boxSegs > 1 ? V.boxSegs : 1);
-    if (V.K == 3) k_dilu_box_pair<T, 3><<<nb, 128, 0, s>>>(V, st, in, out);
-    else k_dilu_box_pair<T, 0><<<nb, 128, 0, s>>>(V, st, in, out);
+    k_dilu_box_pair<T><<<nb, 128, 0, s>>>(V, st, in, out);
     return hipGetLastError();
 }
 
@@ -716,8 +716,8 @@ hipError_t diluApplyFused(const DiluView<T> &V, const SysState *st, int inp, con
     in.v = v;
     if (V.boxLone) {
         const int nb = V.nBoxWaves * (V.boxSegs > 1 ? V.boxSegs : 1);
-        if (inp == kInpP) k_dilu_box_pair<T, 3, kInpP><<<nb, 128, 0, s>>>(V, st, dst, out, in);
-        else k_dilu_box_pair<T, 3, kInpS><<<nb, 128, 0, s>>>(V, st, dst, out, in);
+        if (inp == kInpP) k_dilu_box_pair<T, kInpP><<<nb, 128, 0, s>>>(V, st, dst, out, in);
+        else k_dilu_box_pair<T, kInpS><<<nb, 128, 0, s>>>(V, st, dst, out, in);
         return hipGetLastError();
     }
     using U = typename Bits<T>::U;
