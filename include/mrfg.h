@@ -460,7 +460,8 @@ int mrfg_set_wait_limit(mrfg_ctx *ctx, int polls);
 /* info[0..5] = cells, internal faces, GGI pairs, rows incl. padding,
    64-row slices, DILU waves. */
 int mrfg_layout_info(mrfg_ctx *ctx, int sys, long long *info);
-/* Canonical algorithmic bytes at value size 8 (fp64) or 4 (fp32). */
+/* Canonical algorithmic bytes at value size 8 (fp64) or 4 (fp32); b_spmv counts
+   a column index per face entry, also where the layout needs none. */
 int mrfg_bytes(mrfg_ctx *ctx, int sys, int value_size, double *b_iter, double *b_spmv, double *b_dilu);
 /* Average time (ms) of a plain device-to-device copy of `bytes` bytes over
    `reps` launches (each reads and writes `bytes`): the reference kernel for

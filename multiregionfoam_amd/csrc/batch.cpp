@@ -1635,6 +1635,8 @@ int Batch::traceDilu(long long *out, int maxWaves)
     return nWaves_;
 }
 
+// (the canonical bytes, with a column per face entry: 3-D box rows read none,
+// so a rate from them is higher than what is moved)
 double Batch::bytesSpmv(int sys, int sv) const
 {
     const SystemLayout &L = *lay_.at(sys);

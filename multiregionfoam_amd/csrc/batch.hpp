@@ -368,18 +368,17 @@ private:
     bool boxLone_ = false;   // every box tile alone in its region
     bool factorised_ = false, haveFloat_ = false;
     bool tileLocal32_ = false;   // the FP32 records are those of the tile-local DILU
-    // segments per box tile in the tile-local DILU, each swept by a wave of
-    // its own (a shorter chain of steps, slightly more inner iterations): as
-    // many as keep the lone waves within kTileSegWaves, at most 3.  The waves
-    // may outnumber the CUs several times over: duct3d (135 tiles) takes 3
-    // segments (33.6 ms per mixed solve against 37.1 with 2 and 39.9 with 1;
-    // 4 needed more iterations than they saved), exchanger3 (585 tiles) 3
-    // (362.8 -> 328.6 ms), batch64 2 (656 -> 558 ms; a budget of 16384 waves,
-    // giving it 3, was slower: 590 ms)
-    static constexpr int kTileSegWaves = 8192;
+    // segments per box tile in the tile-local DILU, each swept by a workgroup
+    // of its own (a shorter chain of steps, mostly more inner iterations): as
+    // many as keep the lone workgroups within kTileSegGroups, at most 3.  They
+    // may outnumber the CUs several times over.  Per mixed solve with 1, 2, 3
+    // and 4 segments: duct3d (135 tiles, takes 3) 37.0, 30.6, 30.0 and 28.2
+    // ms; exchanger3 (585, takes 3) 226, 342, 272 and 325 ms, at 468, 631, 548
+    // and 672 iterations; batch64 (takes 2) 506, 433, 466 and 463 ms
+    static constexpr int kTileSegGroups = 8192;
     int tileSegments() const
     {
-        return nBoxWaves_ > 0 ? std::max(1, std::min(3, kTileSegWaves / nBoxWaves_)) : 1;
+        return nBoxWaves_ > 0 ? std::max(1, std::min(3, kTileSegGroups / nBoxWaves_)) : 1;
     }
 
     // structure (shared by both precisions)

@@ -1,6 +1,7 @@
 // DILU (coupled Cholesky preconditioner) on gfx950: factorisation and the
 // forward / backward sweeps of the preconditioner, executed by a schedule of
-// waves (one wavefront per workgroup).
+// chains (one wavefront per workgroup), level groups (a workgroup of up to 16
+// per region) and spread levels (the whole device).
 //
 // Restated arithmetic (per region; interface coefficients are not part of
 // the factor, the coupled preconditioner works on each region's lduMatrix):
@@ -12,7 +13,8 @@
 // their factorisation at the end of this file.
 //
 // Each lane holds one row per step, whose dependencies were computed earlier
-// by the same wave (chains) or workgroup (level groups) and are read from LDS.
+// by the same wave (chains) or workgroup (level groups) and are read from LDS,
+// or by an earlier launch (spread levels).
 // A step of a chain is latency-bound (one LDS round trip plus a short FMA
 // chain), so the kernel keeps memory out of the critical path: each row's
 // record is a few 16-byte chunks, prefetched kPrefetch steps ahead, every
@@ -210,7 +212,8 @@ __global__ __launch_bounds__(64) void k_dilu_wave(DiluView<T> V, const SysState 
 // renumbered along a front (122 levels of up to 957 rows), against what is
 // bound here by one CU's load path (60 bytes a row in FP64, about 64 bytes a
 // clock) and the barrier.  Two regions of a system, or the systems of a batch,
-// run side by side on CUs of their own.
+// run side by side on CUs of their own.  Regions with wide levels are spread
+// over the device instead (layout.cpp, spreadPays).
 //
 // One CU only has so many cache misses in flight: its rows came at 31 GB/s
 // (105 us a sweep of that mesh; 81 us with the helpers below), whatever the
@@ -565,8 +568,8 @@ __device__ __forceinline__ void boxFactor(const DiluView<double> &V, const int32
                 // poll rounds: each reloads this step's values and those
                 // already requested for the next steps, all in flight
                 // together; the later ones come with the last round instead
-                // of a round trip each (145 -> 240 us a factor of the 1.4M
-                // cell duct without)
+                // of a round trip each (a factor of the 1.4M cell duct takes
+                // 145 us, 240 without)
                 for (int spins = 0;; ++spins) {
                     U nb[kFacInAhead], nc[kFacInAhead];
 #pragma unroll
