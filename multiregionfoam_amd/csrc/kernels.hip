@@ -229,32 +229,39 @@ __global__ __launch_bounds__(kFinBlock) void k_finalize(int stage, const SysInfo
 
 // The face terms of a 3-D box tile's row, sequential axis AX: six entries in
 // the order z, y, x lower, x, y, z upper, whose columns follow from the tile.
-// A zero entry (no neighbour) reads the row's own x.  Without the column array
+// An entry without a neighbour is not added.  Without the column array
 // a row reads 80 bytes instead of 104 (40 instead of 64 in FP32): on the 1.4M
 // cell duct the product with its sum takes 33.2 us inside the FP64 solve (40.8
 // before), and the mixed solve 29.2 ms (30.7).
 template <typename T, int AX>
-__device__ inline T spmvBoxRow(const MatView<T> &A, const int (&g)[6], int e0, int lane, int p, T y,
+__device__ inline T spmvBoxRow(const MatView<T> &A, const int (&g)[kSliceGeom], int e0, int lane, int p, T y,
                                const T *__restrict__ x)
 {
     const T *v = A.ellVal + (size_t)e0 * 64 + lane;
     T val[6], xv[6];
 #pragma unroll
     for (int j = 0; j < 6; ++j) val[j] = v[j * 64];
-    const int lg = g[kSgLogTB], TB = 1 << lg, bl = lane & (TB - 1), cl = lane >> lg;
+    const int lg = g[kSgTile] & 0xFF, actB = (g[kSgTile] >> 8) & 0xFF, actC = g[kSgTile] >> 16;
+    const int TB = 1 << lg, bl = lane & (TB - 1), cl = lane >> lg, ia = g[kSgStep] - bl - cl;
     // distances along the tile's axes a (sequential), b, c; lower then upper
     const int d[3][2] = {{-64, 64},
                          {bl > 0 ? -65 : g[kSgPrevB], bl < TB - 1 ? 65 : g[kSgNextB]},
                          {cl > 0 ? -64 - TB : g[kSgPrevC], cl < (64 >> lg) - 1 ? 64 + TB : g[kSgNextC]}};
+    const bool has[3][2] = {{ia > 0, ia < g[kSgNA] - 1},
+                            {bl > 0 || g[kSgPrevB] != 0, bl < actB - 1 || g[kSgNextB] != 0},
+                            {cl > 0 || g[kSgPrevC] != 0, cl < actC - 1 || g[kSgNextC] != 0}};
     // axis (x, y, z) -> tile axis
     constexpr int of[3] = {AX == 0 ? 0 : 1, AX == 1 ? 0 : AX == 0 ? 1 : 2, AX == 2 ? 0 : 2};
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
-        const int dj = j < 3 ? d[of[2 - j]][0] : d[of[j - 3]][1];
-        xv[j] = x[val[j] != T(0) ? p + dj : p];
+        const int k = of[j < 3 ? 2 - j : j - 3], up = j < 3 ? 0 : 1;
+        xv[j] = x[has[k][up] ? p + d[k][up] : p];
     }
 #pragma unroll
-    for (int j = 0; j < 6; ++j) y = y + val[j] * xv[j];
+    for (int j = 0; j < 6; ++j) {
+        const T t = y + val[j] * xv[j];
+        y = has[of[j < 3 ? 2 - j : j - 3]][j < 3 ? 0 : 1] ? t : y;
+    }
     return y;
 }
 
@@ -269,9 +276,10 @@ __device__ inline T spmvRow(const MatView<T> &A, int s, int lane, int p, const T
     // (the slice's, the same for the whole wave: the branch is uniform)
     const int4 *gp = reinterpret_cast<const int4 *>(A.sliceGeom + (size_t)s * kSliceGeom);
     const int4 ga = gp[0], gb = gp[1];
-    const int g[6] = {__builtin_amdgcn_readfirstlane(ga.x), __builtin_amdgcn_readfirstlane(ga.y),
+    const int g[kSliceGeom] = {__builtin_amdgcn_readfirstlane(ga.x), __builtin_amdgcn_readfirstlane(ga.y),
                       __builtin_amdgcn_readfirstlane(ga.z), __builtin_amdgcn_readfirstlane(ga.w),
-                      __builtin_amdgcn_readfirstlane(gb.x), __builtin_amdgcn_readfirstlane(gb.y)};
+                      __builtin_amdgcn_readfirstlane(gb.x), __builtin_amdgcn_readfirstlane(gb.y),
+                      __builtin_amdgcn_readfirstlane(gb.z), __builtin_amdgcn_readfirstlane(gb.w)};
     switch (g[kSgAxis]) {
     case 0: y = spmvBoxRow<T, 0>(A, g, e0, lane, p, y, x); break;
     case 1: y = spmvBoxRow<T, 1>(A, g, e0, lane, p, y, x); break;

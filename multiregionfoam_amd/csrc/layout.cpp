@@ -486,11 +486,18 @@ SystemLayout buildLayout(const CoupledSystem &sys, bool preferLevels)
         auto across = [&](int to, int dStep, int dLane) {
             return m[to] < 0 ? 0 : (L.waveSlice[m[to]] - L.waveSlice[wi] + dStep) * kSlice + dLane;
         };
-        const int g[kSliceGeom] = {m[kBmAxis], __builtin_ctz(TB), across(kBmPrevB, TB - 1, TB - 1),
-                                   across(kBmNextB, 1 - TB, 1 - TB), across(kBmPrevC, TC - 1, TB * (TC - 1)),
-                                   across(kBmNextC, 1 - TC, -TB * (TC - 1)), 0, 0};
-        for (int t = 0; t < L.waveSteps[wi]; ++t)
+        int g[kSliceGeom] = {m[kBmAxis],
+                             __builtin_ctz(TB) | m[kBmActB] << 8 | m[kBmActC] << 16,
+                             across(kBmPrevB, TB - 1, TB - 1),
+                             across(kBmNextB, 1 - TB, 1 - TB),
+                             across(kBmPrevC, TC - 1, TB * (TC - 1)),
+                             across(kBmNextC, 1 - TC, -TB * (TC - 1)),
+                             0,
+                             m[kBmNA]};
+        for (int t = 0; t < L.waveSteps[wi]; ++t) {
+            g[kSgStep] = t;
             std::copy(g, g + kSliceGeom, &L.sliceGeom[(size_t)(L.waveSlice[wi] + t) * kSliceGeom]);
+        }
     }
 
     // ---- per-slice ELL (SpMV) ----

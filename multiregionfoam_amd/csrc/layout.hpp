@@ -88,9 +88,10 @@ enum {
 };
 
 // Per-slice geometry: the sequential axis (-1: not a 3-D box tile, the columns
-// are listed), log2 of TB, and for the rows on the tile's edges the distance to
-// the neighbour's position across it (0: none).
-enum { kSgAxis = 0, kSgLogTB, kSgPrevB, kSgNextB, kSgPrevC, kSgNextC, kSliceGeom = 8 };
+// are listed); log2 of TB, actB << 8 and actC << 16; for the rows on the tile's
+// edges the distance to the neighbour's position across it (0: none); the
+// slice's step of the tile; nA.
+enum { kSgAxis = 0, kSgTile, kSgPrevB, kSgNextB, kSgPrevC, kSgNextC, kSgStep, kSgNA, kSliceGeom = 8 };
 
 struct RegionSchedule {
     std::string kind;                // "box", "chain", "levels" or "spread"

@@ -98,3 +98,27 @@ def test_expired_wait_fails_the_call(gpu):
         with pytest.raises(Exception, match="polls must be"):
             A.set_wait_limit(polls)
     A.close()
+
+
+@pytest.mark.parametrize("n", [(3, 2, 2), (12, 9, 7), (33, 17, 9), (17, 33, 70), (20, 90, 31)],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_spmv_of_values_that_are_not_finite(gpu, n):
+    # a face with a zero coefficient still multiplies its neighbour's value,
+    # and a cell without a neighbour multiplies nothing
+    R = box(n, 8)
+    rng = np.random.default_rng(9)
+    for side in ("lower", "upper"):
+        R[side][rng.random(R["nFaces"]) < 0.3] = 0.0
+    O = ob.OracleSystem.from_arrays([R], [])
+    A = _committed(gpu, [R])
+    x = rng.standard_normal(R["nCells"])
+    x[rng.random(len(x)) < 0.05] = 0.0
+    assert np.array_equal(A.spmv([x]), np.concatenate(O.amul([x])))
+    for k, v in enumerate((np.inf, -np.inf, np.nan)):
+        bad = np.random.default_rng(10 + k).choice(len(x), max(1, len(x) // 300), replace=False)
+        y = x.copy()
+        # the corners too: cells that lack neighbours on three sides
+        y[np.concatenate([bad, [0, len(x) - 1]])] = v
+        want = np.concatenate(O.amul([y]))
+        assert np.array_equal(A.spmv([y]), want, equal_nan=True)
+    A.close()
