@@ -17,8 +17,8 @@ static void check(bool ok, const char *what)
     }
 }
 
-// whether a further holder of `more` gets in beside `held`
-static bool together(int slots, std::vector<int> held, int more)
+// whether a further holder of `more` gets in beside `held`, as `expected`
+static bool together(int slots, std::vector<int> held, int more, bool expected)
 {
     auto *gate = new SweepGate(slots);   // (kept: a waiting thread may outlive this call)
     for (int t : held) gate->acquire(t);
@@ -27,25 +27,25 @@ static bool together(int slots, std::vector<int> held, int more)
         gate->acquire(more);
         *in = true;
     });
-    for (int k = 0; k < 100 && !*in; ++k) std::this_thread::sleep_for(std::chrono::milliseconds(2));
+    for (int k = 0; k < (expected ? 10000 : 100) && !*in; ++k) std::this_thread::sleep_for(std::chrono::milliseconds(2));
     const bool yes = *in;
     if (yes) gate->release(more);
     // everyone gets in once the others are done
     for (int t : held) gate->release(t);
     th.join();
-    return yes;
+    return yes == expected;
 }
 
 int main()
 {
-    check(together(96, {}, 5000), "the first always");
-    check(together(96, {5000}, 95), "beside a larger one, with a slot left");
-    check(!together(96, {5000}, 96), "no slot left");
-    check(together(96, {38, 38}, 38), "three of 300 tiles");
-    check(!together(96, {38, 38, 38}, 38), "four of 300 tiles");
-    check(together(96, {38, 38}, 5000), "a large one beside small ones");
-    check(!together(96, {48, 48}, 5000), "small ones that fill an XCD");
-    check(together(96, {5000, 20}, 0), "no box tiles");
+    check(together(96, {}, 5000, true), "the first always");
+    check(together(96, {5000}, 95, true), "beside a larger one, with a slot left");
+    check(together(96, {5000}, 96, false), "no slot left");
+    check(together(96, {38, 38}, 38, true), "three of 300 tiles");
+    check(together(96, {38, 38, 38}, 38, false), "four of 300 tiles");
+    check(together(96, {38, 38}, 5000, true), "a large one beside small ones");
+    check(together(96, {48, 48}, 5000, false), "small ones that fill an XCD");
+    check(together(96, {5000, 20}, 0, true), "no box tiles");
     // many threads: the rule holds at all times and all get through
     SweepGate gate(96);
     std::mutex m;

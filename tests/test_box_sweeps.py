@@ -65,15 +65,15 @@ def _committed(gpu, regions):
 
 
 def test_wait_limit_is_of_one_wait(gpu):
-    # two flat tiles of 30000 steps: the second waits for a few steps of the
-    # first at a time, some 4000 polls in the whole sweep
-    regions = [box((30000, 66, 1), 4)]
+    # two flat tiles of 60000 steps: the second waits for a few steps of the
+    # first at a time, some 3000 polls in the whole sweep
+    regions = [box((60000, 66, 1), 4)]
     A = _committed(gpu, regions)
     assert len(set(A.dilu_tiles())) > 1
     rD = A.dilu_factor()
     r = [np.random.default_rng(5).standard_normal(R["nCells"]) for R in regions]
     w = A.precondition(r)
-    A.set_wait_limit(500)
+    A.set_wait_limit(1000)
     assert np.array_equal(A.dilu_factor(), rD)
     assert np.array_equal(A.precondition(r), w)
     A.close()
