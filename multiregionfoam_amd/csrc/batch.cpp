@@ -521,8 +521,7 @@ void Batch::setSystems(const std::vector<const CoupledSystem *> &systems,
         spread.insert(spread.end(), lv.begin(), lv.end());
         spreadLevels_.push_back((int)spread.size());
     }
-    if (spread.empty()) spread.push_back(SpreadSlice{});
-    spread_.upload(spread, stream_);
+    if (!spread.empty()) spread_.upload(spread, stream_);
     if (groups.empty()) groups.push_back(LevelGroup{});
     if (rounds.empty()) rounds.push_back(LevelRound{0, 0});
     groups_.upload(groups, stream_);
